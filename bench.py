@@ -60,7 +60,7 @@ sys.path.insert(0, ROOT)
 HBM_PEAK_GBS = 8000.0
 KCLASS = {0: "k_dst_x (row pass, time step)", 1: "k_dst_y (column pass, time step)",
           2: "k_dst_x (batched row pass, Schur assembly)", 3: "k_dst_y (batched column pass, Schur assembly)",
-          4: "k_gmres_coopw (one dense GMRES solve over P workgroups of one XCD; k_gmres_coop for nf <= 256, "
+          4: "k_gmres_coopw (one dense GMRES solve over P workgroups of one XCD; "
              "k_gmres_dense in one workgroup where no split fits)"}
 FP64_PEAK_TFLOPS = 78.6
 
@@ -173,8 +173,8 @@ def run_gpu(args):
                               3: "cooperative (nf <= 1024)"}[form]
         roof["workgroups"] = wgs
         roof["exchange"] = {0: "none", 1: "through one XCD's L2", 2: "device scope"}[xch]
-        roof["limited_by"] = ("latency: three grid barriers and a few dependent L2 round trips per Arnoldi step "
-                              "across the workgroups of one XCD; S and the basis stay on chip, so HBM is idle")
+        roof["limited_by"] = ("latency: two or three exchanges through L2 per Arnoldi step and the short dependent "
+                              "products between them; S and the basis stay on chip, so HBM is idle")
         roof["algorithmic_bytes"] = ("per Arnoldi step: S (nf^2 doubles), basis vectors 0..j read twice by "
                                      "classical Gram-Schmidt, the new vector written; b and x per solve")
     roof["other_classes"] = [summary(kc) for kc in classes if kc != dom]

@@ -698,28 +698,13 @@ void gmres_dense(hipStream_t st, int nf, int kmax, int maxit, const double* S, c
 }
 
 // ------------------------------------------------------------------------
-// The same dense solve spread over P workgroups of one XCD.  Workgroup c
-// owns rows [c R, c R + R) of S (in registers: four rows by kCoopColQ
-// columns per thread) and those rows of every Krylov vector (in LDS), so
-// neither S nor the basis is re-read from L2.  Per Arnoldi step the
-// workgroups exchange, through L2 and two grid barriers, the partial CGS
-// coefficients of their rows, then the partial squared norm and their rows
-// of w.  Every workgroup sums the partials of all workgroups in the same
-// order and runs the rotations, tests and back substitution on identical
-// values, so all take the same branches; each updates its rows of x.  The
-// launch has 8P workgroups, dealt by the dispatcher to the 8 XCDs in turn;
-// the P on the XCD the host names take part (coop_rank), so a solve keeps
-// to one XCD's CUs and L2 and solves on different XCDs run side by side.
-// The exchanged values are device-scope atomic stores and loads (coherent
-// without cache write-backs); the barrier waits are bounded: on a timeout
-// every workgroup leaves with reason -3.
+// The same dense solve spread over P workgroups of one XCD (k_gmres_coopw,
+// below).  The launch has P workgroups per XCD, dealt by the dispatcher to
+// the XCDs in turn; the P on the XCD the host names take part, so
+// a solve keeps to one XCD's CUs and L2 and solves on different XCDs run side
+// by side.  All waits are bounded: on a timeout every workgroup leaves with
+// reason -3.
 // ------------------------------------------------------------------------
-// Thread layout of the matrix-vector product and of w -= V h: wavefront q
-// of the 16 owns local rows 4q .. 4q+3 (R <= 64), lane l the columns
-// l, l + 64, ... (nf <= 64 kCoopColQ); each lane's four row partials are
-// summed over the wavefront by gc_reduce4.
-constexpr int kCoopColQ = 4;
-constexpr int kCoopRowsPer16 = 4;  // local rows per 16-lane group in the CGS dots: R <= 64
 constexpr long kCoopSpin = 1L << 22;
 
 // The barrier block of a cooperative solve (unsigned words, cleared before
@@ -732,37 +717,6 @@ static_assert(kClaimSlot < 2 * kCoopSyncDoubles, "barrier block too small");
 
 // The XCD this wavefront runs on (HW_REG_XCC_ID, bits 3:0).
 __device__ __forceinline__ unsigned gw_xcc_id() { return __builtin_amdgcn_s_getreg((3 << 11) | (0 << 6) | 20) & 0xFu; }
-
-// The rank of this workgroup in a cooperative solve of P workgroups, or -1
-// if it takes no part.  xcd < 0: workgroups 0, 8, 16, ... (one XCD when the
-// dispatcher starts the launch's round on it); xcd >= 0: the first P
-// workgroups that run on XCD xcd (XCC_ID), ranked in the order they claim.
-// A launch of 8P workgroups puts P on every XCD.
-__device__ __forceinline__ int coop_rank(unsigned* sync, int P, int xcd, int* s_c) {
-  if (xcd < 0) return blockIdx.x % 8 == 0 && (int)(blockIdx.x / 8) < P ? (int)(blockIdx.x / 8) : -1;
-  if (threadIdx.x == 0)
-    *s_c = gw_xcc_id() == (unsigned)xcd
-               ? (int)__hip_atomic_fetch_add(sync + kClaimSlot, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-               : P;
-  __syncthreads();
-  const int c = *s_c;
-  return c < P ? c : -1;
-}
-
-// Before a cooperative launch: the barrier block cleared and the status set
-// to reason -3, which stays if no workgroup takes part.
-__global__ void k_coop_prep(unsigned* sync, GmresDev* s) {
-  if (threadIdx.x < 2 * kCoopSyncDoubles) sync[threadIdx.x] = 0u;
-  if (threadIdx.x == 0) {
-    s->reason = -3;
-    s->its = 0;
-  }
-}
-
-static void coop_prep(hipStream_t st, double* ws, GmresDev* s) {
-  hipLaunchKernelGGL(k_coop_prep, dim3(1), dim3(2 * kCoopSyncDoubles), 0, st, reinterpret_cast<unsigned*>(ws), s);
-  IB_LAUNCH_CHECK();
-}
 
 __global__ void k_xcc_probe(unsigned* ids) {
   if (threadIdx.x == 0) ids[blockIdx.x] = gw_xcc_id();
@@ -794,50 +748,25 @@ std::vector<int> gmres_xcc_ids(hipStream_t st) {
   return ids;
 }
 
-struct GmCoopArgs {
-  int nf, kmax, maxit, P, R;
-  int xcd;        // the XCD whose workgroups take part (-1: workgroups 0, 8, 16, ...)
-  int bsc;        // Hessenberg columns per back-substitution chunk
-  const double* S;
-  const double* b;
-  double* x;
-  GmresDev* s;
-  double rtol, atol;
-  unsigned* sync;  // [0] error, [8 + c] barriers passed by workgroup c
-  double* dots;    // P x (kmax + 2) partial CGS coefficients
-  double* norms;   // P x 4 partial squared norms
-  double* wfull;   // nf: w (or r) rows of every workgroup
-  double* H;       // P x (kmax + 1) x kmax: one Hessenberg copy per workgroup
-};
-
-// A value another workgroup wrote before the last grid barrier.  An atomic
-// load is always a vector memory access (served by L2 once the barrier has
-// invalidated L1); a plain load of a uniform address could be served by the
-// scalar cache, which the barrier does not refresh.
-__device__ __forceinline__ double gc_ld(const double* p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// v + the value of the lane 16 (32) further, modulo 32 (64): the rows of 16
+// lanes (the halves of the wavefront) are swapped between two copies of v, and
+// every lane adds the lower row's value and the higher's, so both lanes of a
+// pair get the same bits
+__device__ __forceinline__ double gm_add_xor16(double v) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  const unsigned lo = (unsigned)b, hi = (unsigned)(b >> 32);
+  const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+  const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+  return __longlong_as_double((long long)(((unsigned long long)h[0] << 32) | l[0])) +
+         __longlong_as_double((long long)(((unsigned long long)h[1] << 32) | l[1]));
 }
-// A value other workgroups read after the next grid barrier (coherent at
-// device scope without a cache write-back).
-__device__ __forceinline__ void gc_st(double* p, double v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// The sum over q = 0..P-1 (in that order) of p[q * stride], values other
-// workgroups wrote before the last grid barrier: the loads go out in
-// batches of 8 (clamped indices) before any of them is used, so a batch
-// costs one memory round trip instead of one per value.
-__device__ __forceinline__ double gc_sum(const double* p, long stride, int P) {
-  double h = 0.0;
-  for (int q0 = 0; q0 < P; q0 += 8) {
-    double v[8];
-#pragma unroll
-    for (int q = 0; q < 8; ++q) v[q] = gc_ld(p + (long)min(q0 + q, P - 1) * stride);
-#pragma unroll
-    for (int q = 0; q < 8; ++q)
-      if (q0 + q < P) h += v[q];
-  }
-  return h;
+__device__ __forceinline__ double gm_add_xor32(double v) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  const unsigned lo = (unsigned)b, hi = (unsigned)(b >> 32);
+  const auto l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+  const auto h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+  return __longlong_as_double((long long)(((unsigned long long)h[0] << 32) | l[0])) +
+         __longlong_as_double((long long)(((unsigned long long)h[1] << 32) | l[1]));
 }
 
 // Every lane of a wavefront holds partial sums v0..v3 of four rows; returns
@@ -857,13 +786,8 @@ __device__ __forceinline__ double gc_reduce4(double v0, double v1, double v2, do
   k += gm_dpp<0x4E>(hi ? k0 : k1);
   k += gm_dpp<0x124>(k);
   k += gm_dpp<0x128>(k);
-  k += __shfl_xor(k, 16);
-  k += __shfl_xor(k, 32);
-  return k;
+  return gm_add_xor32(gm_add_xor16(k));
 }
-// the local row whose sum gc_reduce4 leaves in lane l of wavefront q
-__device__ __forceinline__ int gc_reduce4_row(int q, int l) { return 4 * q + (((l & 1) << 1) | ((l >> 1) & 1)); }
-
 // Wait until every vector memory operation this wavefront issued has
 // completed; for the device-scope stores above that means they have
 // reached the coherent level.  A workgroup-scope release fence does not
@@ -871,406 +795,61 @@ __device__ __forceinline__ int gc_reduce4_row(int q, int l) { return 4 * q + (((
 // another wavefront's flag store could overtake this wavefront's data.
 __device__ __forceinline__ void gc_wait_stores() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
-// Grid barrier number k (1, 2, ...) over the P workgroups.  Each
-// workgroup's values are device-scope atomic stores.  Every wavefront
-// waits for its own stores to complete (gc_wait_stores) before the
-// workgroup barrier, so when wavefront 0 then publishes flag[c] = k every
-// store of workgroup c is visible at device scope; wavefront 0 polls the P
-// flags (one lane each) until all have reached k, and the others wait at
-// the second workgroup barrier, after which their device-scope loads see
-// the other workgroups' values.  Bounded: on a timeout (or another
-// workgroup's) the error word is set and every workgroup leaves.
-__device__ __forceinline__ bool gc_sync(unsigned* sync, int P, int c, unsigned k, int* s_err) {
-  gc_wait_stores();
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  __syncthreads();
-  if (threadIdx.x < 64) {
-    unsigned* err = sync;
-    unsigned* fl = sync + 8;
-    const int lane = threadIdx.x;
-    if (lane == 0) __hip_atomic_store(fl + c, k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    long n = 0;
-    while (true) {
-      const unsigned v = lane < P ? __hip_atomic_load(fl + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : k;
-      if (__all(v >= k)) break;
-      if (__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u || ++n > kCoopSpin) {
-        if (lane == 0) {
-          __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          *s_err = 1;
-        }
-        break;
-      }
-      __builtin_amdgcn_s_sleep(1);
-    }
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-  }
-  __syncthreads();
-  return *s_err == 0;
-}
-
-__global__ void __launch_bounds__(kGmT) k_gmres_coop(GmCoopArgs a) {
-  __shared__ int s_c;
-  const int c = coop_rank(a.sync, a.P, a.xcd, &s_c);
-  if (c < 0) return;
-  extern __shared__ double dyn[];
-  const int nf = a.nf, kmax = a.kmax, ld = kmax + 1, T = kGmT, R = a.R;
-  const int r0 = c * R, Rc = max(0, min(nf, r0 + R) - r0);
-  double* vfull = dyn;                          // nf: the vector being multiplied
-  double* Vl = vfull + nf;                      // (kmax + 1) R: local rows of the basis, vector j at Vl + j R
-  double* wl = Vl + (size_t)(kmax + 1) * R;     // R: local rows of w
-  double* part = wl + R;                        // T
-  double* hcol = part + T;                      // kmax + 2
-  double* lcc = hcol + kmax + 2;                // kmax
-  double* lss = lcc + kmax;                     // kmax
-  double* grs = lss + kmax;                     // kmax + 1
-  double* yv = grs + kmax + 1;                  // kmax + 1
-  double* hrot = yv + kmax + 1;                 // kmax + 2: the new Hessenberg column after the rotations
-  __shared__ double red[kGmT / 64];
-  __shared__ double s_val[2];
-  __shared__ int s_flag[2];
-  __shared__ int s_err;
-  if (threadIdx.x == 0) s_err = 0;
-  double* Hc = a.H + (size_t)c * ld * kmax;
-  // S[r0 + 4 wq + k][ln + 64 q] in registers (0 outside the matrix)
-  const int wq = threadIdx.x >> 6, ln = threadIdx.x & 63;
-  double sreg[4][kCoopColQ];
-#pragma unroll
-  for (int k = 0; k < 4; ++k)
-#pragma unroll
-    for (int q = 0; q < kCoopColQ; ++q) {
-      const int row = 4 * wq + k, col = ln + 64 * q;
-      sreg[k][q] = row < Rc && col < nf ? a.S[(long)col * nf + r0 + row] : 0.0;
-    }
-  __syncthreads();
-
-  // wl = S[local rows] vfull (ends with a barrier)
-  auto matvec = [&]() {
-    const int q4 = gm_opaque(threadIdx.x) >> 6, l = gm_opaque(threadIdx.x) & 63;
-    if (4 * q4 < Rc) {  // uniform over the wavefront
-      double vv[kCoopColQ];
-#pragma unroll
-      for (int q = 0; q < kCoopColQ; ++q) vv[q] = vfull[min(l + 64 * q, nf - 1)];
-      double acc[4];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        acc[k] = 0.0;
-#pragma unroll
-        for (int q = 0; q < kCoopColQ; ++q) acc[k] += sreg[k][q] * vv[q];  // sreg is 0 past the matrix
-      }
-      const double sum = gc_reduce4(acc[0], acc[1], acc[2], acc[3]);
-      const int row = gc_reduce4_row(q4, l);
-      if (l < 4 && row < Rc) wl[row] = sum;
-    }
-    __syncthreads();
-  };
-
-  // the previous rotations applied to the new column (KSPGMRESUpdateHessenberg)
-  // as an affine-recurrence scan, 64 rotations at a time, by one whole
-  // wavefront: hrot[j] for j < it, and hrot[it] = the entry the new rotation
-  // acts on; hcol keeps the unrotated CGS coefficients
-  auto rotate_prev = [&](int it, int lane) {
-    double carry = hcol[0];
-    for (int base = 0; base < it; base += 64) {
-      const int j = base + lane;
-      const bool act = j < it;
-      const double cj0 = act ? lcc[j] : 1.0, sj = act ? lss[j] : 0.0, hn = act ? hcol[j + 1] : 0.0;
-      double A = -sj, B = cj0 * hn;
-      gm_affine_scan(A, B);
-      const double cnext = A * carry + B;
-      const double cj = gm_shift_up1(cnext, carry);
-      if (act) hrot[j] = cj0 * cj + sj * hn;
-      carry = gm_readlane(cnext, min(63, it - 1 - base));
-    }
-    if (lane == 0) hrot[it] = carry;
-  };
-  // the last wavefront owns no rows of the update w -= V h when R <= 60: it
-  // runs the scan while the others update w
-  const bool scan_early = 4 * (T / 64 - 1) >= Rc;
-
-  int its = 0, reason = 0, first = 1;
-  unsigned bk = 0;  // grid barriers passed
-  double rn0 = 0.0, ttol = 0.0;
-  while (true) {
-    // ---- cycle start: r = b - S x (x gathered from every workgroup's rows)
-    for (int i = gm_opaque(threadIdx.x); i < nf; i += T) vfull[i] = gc_ld(a.x + i);
-    __syncthreads();
-    matvec();
-    double pr = 0.0, pb = 0.0;
-    for (int r = gm_opaque(threadIdx.x); r < Rc; r += T) {
-      const double bv = a.b[r0 + r];
-      const double rv = bv - wl[r];
-      gc_st(a.wfull + r0 + r, rv);
-      pr += rv * rv;
-      pb += bv * bv;
-    }
-    pr = gm_block_sum2(pr, red, T);
-    pb = gm_block_sum2(pb, red, T);
-    if (threadIdx.x == 0) {
-      gc_st(a.norms + c * 4 + 1, pr);
-      gc_st(a.norms + c * 4 + 2, pb);
-    }
-    if (!gc_sync(a.sync, a.P, c, ++bk, &s_err)) break;
-    const double sr = gc_sum(a.norms + 1, 4, a.P), sb = gc_sum(a.norms + 2, 4, a.P);
-    const double res0 = sqrt(sr), bn = sqrt(sb);
-    if (first) {
-      rn0 = bn > 0.0 ? bn : res0;
-      ttol = fmax(a.rtol * rn0, a.atol);
-      first = 0;
-    }
-    if (res0 == 0.0 || res0 <= ttol) reason = 1;
-    else if (res0 >= 1e4 * rn0) reason = -1;
-    if (reason) break;
-    if (threadIdx.x == 0) grs[0] = res0;
-    for (int i = gm_opaque(threadIdx.x); i < nf; i += T) vfull[i] = gc_ld(a.wfull + i) / res0;
-    for (int r = gm_opaque(threadIdx.x); r < Rc; r += T) Vl[r] = gc_ld(a.wfull + r0 + r) / res0;
-    __syncthreads();
-    int it = 0;
-    bool ok = true;
-    while (true) {
-      matvec();  // w = S v_it, local rows
-      // partial CGS coefficients <w, v_j>, j = 0..it, over the local rows:
-      // 16 lanes per coefficient
-      {
-        const int t = gm_opaque(threadIdx.x), sub = t & 15;
-        double wr[kCoopRowsPer16];  // rows sub, sub + 16, ... of w (R <= 16 kCoopRowsPer16)
-#pragma unroll
-        for (int q = 0; q < kCoopRowsPer16; ++q) wr[q] = sub + 16 * q < Rc ? wl[sub + 16 * q] : 0.0;
-        for (int j = t >> 4; j <= it; j += T / 16) {
-          double p = 0.0;
-#pragma unroll
-          for (int q = 0; q < kCoopRowsPer16; ++q)
-            if (sub + 16 * q < Rc) p += wr[q] * Vl[(long)j * R + sub + 16 * q];
-          p = gm_row_sum16(p);
-          if (sub == 0) gc_st(a.dots + (long)c * (kmax + 2) + j, p);
-        }
-      }
-      if (!gc_sync(a.sync, a.P, c, ++bk, &s_err)) {
-        ok = false;
-        break;
-      }
-      for (int j = gm_opaque(threadIdx.x); j <= it; j += T) hcol[j] = gc_sum(a.dots + j, kmax + 2, a.P);
-      __syncthreads();
-      // w -= sum_j h_j v_j on the local rows (wavefront q4: rows 4 q4 ..
-      // 4 q4 + 3, lane l: j = l, l + 64, ...); partial ||w||^2; w rows out
-      {
-        const int q4 = gm_opaque(threadIdx.x) >> 6, l = gm_opaque(threadIdx.x) & 63;
-        double pn = 0.0;
-        if (4 * q4 < Rc) {  // uniform over the wavefront
-          const int rb = 4 * q4;
-          const bool ok1 = rb + 1 < Rc, ok2 = rb + 2 < Rc, ok3 = rb + 3 < Rc;
-          double acc0 = 0.0, acc1 = 0.0, acc2 = 0.0, acc3 = 0.0;
-          for (int j = l; j <= it; j += 64) {
-            const double hj = -hcol[j];
-            const double* vj = Vl + (long)j * R + rb;
-            acc0 += hj * vj[0];
-            acc1 += hj * (ok1 ? vj[1] : 0.0);
-            acc2 += hj * (ok2 ? vj[2] : 0.0);
-            acc3 += hj * (ok3 ? vj[3] : 0.0);
-          }
-          const double sum = gc_reduce4(acc0, acc1, acc2, acc3);
-          const int row = gc_reduce4_row(q4, l);
-          if (l < 4 && row < Rc) {
-            const double wn = wl[row] + sum;
-            wl[row] = wn;
-            gc_st(a.wfull + r0 + row, wn);
-            pn = wn * wn;
-          }
-        } else if (scan_early && q4 == T / 64 - 1) {
-          rotate_prev(it, l);
-        }
-        pn = gm_block_sum2(pn, red, T);
-        if (threadIdx.x == 0) gc_st(a.norms + c * 4, pn);
-      }
-      if (!gc_sync(a.sync, a.P, c, ++bk, &s_err)) {
-        ok = false;
-        break;
-      }
-      // this thread's entries of the new vector (full and local rows), loaded
-      // with the norm partials so that both take one memory round trip
-      const int t0 = gm_opaque(threadIdx.x);
-      const double wpre = t0 < nf ? gc_ld(a.wfull + t0) : 0.0;
-      const double wpre_l = t0 < Rc ? gc_ld(a.wfull + r0 + t0) : 0.0;
-      const double tt = sqrt(gc_sum(a.norms, 4, a.P));
-      if (gm_opaque(threadIdx.x) < 64) {
-        const int lane = gm_opaque(threadIdx.x);
-        if (!scan_early) rotate_prev(it, lane);
-        if (lane == 0) {
-          hrot[it + 1] = tt;
-          // tt < min(|tt / grs[it]|, 1e-30) (KSPGMRESCycle's happy-breakdown
-          // test); the quotient is needed only when tt < 1e-30
-          const int hap = tt < 1e-30 && tt < fabs(tt / grs[it]);
-          double res;
-          if (!hap) {
-            const double t1 = sqrt(hrot[it] * hrot[it] + hrot[it + 1] * hrot[it + 1]);
-            const double cc = hrot[it] / t1, sn = hrot[it + 1] / t1;
-            lcc[it] = cc;
-            lss[it] = sn;
-            grs[it + 1] = -sn * grs[it];
-            grs[it] = cc * grs[it];
-            hrot[it] = cc * hrot[it] + sn * hrot[it + 1];
-            res = fabs(grs[it + 1]);
-          } else {
-            res = 0.0;
-          }
-          int rs = 0;
-          if (res <= ttol) rs = 1;
-          else if (res >= 1e4 * rn0) rs = -1;
-          if (hap && !rs) rs = 1;
-          s_flag[0] = rs;
-          s_flag[1] = hap;
-          s_val[0] = tt;
-        }
-      }
-      __syncthreads();
-      reason = s_flag[0];
-      const int hap = s_flag[1];
-      for (int j = gm_opaque(threadIdx.x); j <= it + 1; j += T) Hc[(long)it * ld + j] = hrot[j];
-      if (!hap) {
-        const double inv = 1.0 / s_val[0];
-        if (t0 < nf) vfull[t0] = wpre * inv;
-        for (int i = t0 + T; i < nf; i += T) vfull[i] = gc_ld(a.wfull + i) * inv;
-        if (t0 < Rc) Vl[(long)(it + 1) * R + t0] = wpre_l * inv;
-      }
-      ++it;
-      ++its;
-      __syncthreads();
-      if (reason || it >= kmax || its >= a.maxit) break;
-    }
-    if (!ok) break;
-    // ---- KSPGMRESBuildSoln: back substitution on this workgroup's copy of
-    // the rotated Hessenberg (chunks staged in LDS, the serial sweep by one
-    // wavefront), then x += V y on the local rows
-    const int top = it - 1;
-    for (int j = gm_opaque(threadIdx.x); j <= top; j += T) yv[j] = grs[j];
-    for (int k1 = top; k1 >= 0; k1 -= a.bsc) {
-      const int k0 = k1 - a.bsc + 1 < 0 ? 0 : k1 - a.bsc + 1;
-      const int nc = k1 - k0 + 1;
-      __syncthreads();
-      for (int q = gm_opaque(threadIdx.x); q < nc * (k1 + 1); q += T) {
-        const int cq = q / (k1 + 1), rr = q - cq * (k1 + 1);
-        part[(long)cq * ld + rr] = Hc[(long)(k0 + cq) * ld + rr];
-      }
-      __syncthreads();
-      if (threadIdx.x < 64) {
-        const int lane = threadIdx.x;
-        for (int k = k1; k >= k0; --k) {
-          const double* col = part + (long)(k - k0) * ld;
-          const double yk = yv[k] / col[k];
-          for (int j = lane; j < k; j += 64) yv[j] = yv[j] - col[j] * yk;
-          if (lane == 0) yv[k] = yk;
-          __builtin_amdgcn_wave_barrier();
-        }
-      }
-    }
-    __syncthreads();
-    for (int r = gm_opaque(threadIdx.x); r < Rc; r += T) {
-      double acc = 0.0;
-      for (int j = 0; j <= top; ++j) acc += yv[j] * Vl[(long)j * R + r];
-      gc_st(a.x + r0 + r, gc_ld(a.x + r0 + r) + acc);
-    }
-    if (reason) break;
-    if (its >= a.maxit) {
-      reason = -2;
-      break;
-    }
-    if (!gc_sync(a.sync, a.P, c, ++bk, &s_err)) break;  // every workgroup's rows of x before the next residual
-  }
-  if (threadIdx.x == 0) {
-    if (s_err) {
-      a.s->reason = -3;
-      a.s->its = its;
-    } else if (c == 0) {
-      a.s->its = its;
-      a.s->reason = reason;
-      a.s->rn0 = rn0;
-      a.s->ttol = ttol;
-    }
-  }
-}
-
-// dynamic LDS of k_gmres_coop (doubles): vfull nf, Vl (kmax+1) R, wl R,
-// part kGmT, hcol kmax+2, lcc/lss kmax each, grs/yv kmax+1 each, hrot kmax+2
-static size_t coop_lds(int nf, int kmax, int R) {
-  return sizeof(double) * ((size_t)nf + (size_t)(kmax + 1) * R + R + kGmT + (size_t)6 * kmax + 6);
-}
-
-bool gmres_coop_plan(int nf, int kmax, size_t max_lds, int* P, int* R) {
-  static const int cand[] = {2, 4, 8, 16, 32};
-  if (nf > 64 * kCoopColQ) return false;
-  for (int p : cand) {
-    const int r = (nf + p - 1) / p;
-    if (r < 1 || r > 16 * kCoopRowsPer16 || r > 4 * (kGmT / 64) || (p - 1) * r >= nf) continue;
-    if (kGmT / (kmax + 1) < 1) continue;  // back-substitution chunk in the part buffer
-    if (coop_lds(nf, kmax, r) + 1024 > max_lds) continue;
-    *P = p;
-    *R = r;
-    return true;
-  }
-  return false;
-}
-
-size_t gmres_coop_ws(int nf, int kmax, int P) {
-  return kCoopSyncDoubles + (size_t)P * (kmax + 2) + (size_t)4 * P + (size_t)nf + (size_t)P * (kmax + 1) * kmax;
-}
-
-void gmres_coop(hipStream_t st, int nf, int kmax, int maxit, int P, int R, const double* S, const double* b, double* x,
-                GmresDev* s, double rtol, double atol, double* ws, int xcd, int nxcd) {
-  GmCoopArgs a{};
-  a.nf = nf; a.kmax = kmax; a.maxit = maxit; a.P = P; a.R = R; a.xcd = xcd;
-  a.bsc = kGmT / (kmax + 1);
-  a.S = S; a.b = b; a.x = x; a.s = s; a.rtol = rtol; a.atol = atol;
-  a.sync = reinterpret_cast<unsigned*>(ws);
-  a.dots = ws + kCoopSyncDoubles;
-  a.norms = a.dots + (size_t)P * (kmax + 2);
-  a.wfull = a.norms + (size_t)4 * P;
-  a.H = a.wfull + nf;
-  // barrier words cleared by a kernel (a memset node misbehaves on graph replays)
-  coop_prep(st, ws, s);
-  // an ordinary launch: the barrier is the kernel's own (no runtime grid
-  // synchronisation resources), P workgroups per XCD of which the P on XCD
-  // xcd stay (8P and workgroups 0, 8, 16, ... with xcd < 0), one per CU; a
-  // workgroup that is not resident in time makes the others leave with
-  // reason -3 instead of waiting for ever
-  const int nwg = (xcd < 0 ? 8 : std::max(nxcd, 1)) * P;
-  hipLaunchKernelGGL(k_gmres_coop, dim3(nwg), dim3(kGmT), coop_lds(nf, kmax, R), st, a);
-  IB_LAUNCH_CHECK();
-}
-
 // ------------------------------------------------------------------------
-// The dense solve over P workgroups of one XCD for larger systems: nf <=
-// 1024 and Krylov spaces of up to 1024 vectors (full GMRES of the airfoil +
-// flap system, nf = 800, restart 1000).  The same PETSc iteration as
-// k_gmres_coop, laid out for up to 32 rows per workgroup and long Krylov
-// spaces:
-//  * wavefront q owns local rows 2q and 2q+1; lane l holds S[row][l + 64k],
-//    k < CQ, in registers (nf <= 64 CQ), and gw_reduce2 sums a row pair over
-//    the wavefront;
+// The dense solve over P workgroups of one XCD: nf <= 1024 and Krylov spaces
+// of up to 1024 vectors (full GMRES of the airfoil + flap system, nf = 800,
+// restart 1000, over 32 workgroups; the hinged plate, nf = 202, over 4).
+// Workgroup c owns rows [c R, c R + R) of S and of every Krylov vector:
+//  * wavefront q owns RW local rows; lane l holds S[row][l + 64k], k < CQ, in
+//    registers (nf <= 64 CQ), and the row sums go over the wavefront with DPP;
 //  * the local rows of the basis are stored row-major in LDS (row r of
 //    vector j at Vl[r NL + j]), so thread j forms the partial CGS coefficient
 //    of vector j from conflict-free LDS reads, and the update w -= V h reads
 //    consecutive j across the lanes; vectors j >= NL (past the LDS) are kept
 //    in HBM in the same layout;
-//  * the CGS coefficients are reduced and scattered: workgroup c sums the P
-//    partials of coefficients c, c + P, ... in a fixed butterfly order and
-//    publishes them, and after a third grid barrier every workgroup loads
-//    all of them, so all hold identical h and take the same branches;
-//  * the exchange goes through the L2 of the one XCD the workgroups share
-//    (checked with HW_REG_XCC_ID at the start; device scope otherwise);
-//  * the Givens step needs only entry it of the new column after the
-//    previous rotations, which is sum_j alpha_j h_j with alpha updated as
-//    [-s_it alpha, c_it] after each step: one more term in the block
-//    reduction of the norm, instead of a serial scan over the rotations;
-//  * only workgroup 0 keeps the Hessenberg matrix (in HBM, unrotated, with
-//    the rotated diagonal beside it).  At the end of a cycle it applies the
-//    rotations to every column (one thread per column), runs the back
-//    substitution in blocks of kCwBlk columns (diagonal block by one
-//    wavefront from LDS, the rows above by all threads) and publishes y;
-//    every workgroup then adds V y to its rows of x.
+//  * only workgroup 0 keeps the Hessenberg matrix (in HBM, unrotated, row by
+//    row) and runs the back substitution at the end of a cycle.
+//
+// What bounds it is latency: an Arnoldi step is a chain of small products
+// joined by exchanges through L2.  So an exchanged value is its own flag: the
+// buffers hold kUnset (a signalling NaN, which no arithmetic result is) where
+// nothing has been published, a reader polls the value itself until it is
+// there, and no barrier, store wait or second load stands between a
+// workgroup's last product and its neighbours' next one.  A step has three
+// exchanges: the partial CGS coefficients (x1), their sums (x2: workgroup c
+// sums coefficients c, c + P, ...; left out while every workgroup can load
+// all partials in two loads per thread) and the rows of the new vector u
+// (x3).  Everything that is not on that chain runs beside it:
+//  * u is exchanged and multiplied unnormalised (S v = S u / |u|), and every
+//    workgroup has the whole of it, so |u| is the last wavefront's, the same
+//    bits in every workgroup, while the others form S u;
+//  * the Givens step and the stopping tests are the last wavefront's too,
+//    while the others form the dot products of S v.  A step's coefficients are
+//    therefore on their way before it is known whether the step before
+//    converged; after the last one they are not used;
+//  * entry it of the new column after the previous rotations is
+//    sum_j alpha_j h_j with alpha updated as [-s_it alpha, c_it], one dot
+//    product; the stored columns are rotated at the cycle's end.
+// Each buffer has three copies, used in turn.  A workgroup clears what it
+// published in step s once it has published its rows of step s + 1 (its x2 of
+// that step was complete, which takes every workgroup's x1 of step s + 1, and
+// each published that after it had read all of step s), and waits for these
+// stores before it publishes its rows of step s + 2; a reader comes back to
+// the copy in step s + 3, after it has read all rows of step s + 2.  The clears
+// thus run while the rows of step s + 1 travel.
+//
+// Microseconds per Arnoldi step (events around the launches, start-up and
+// back substitution included), with grid barriers around each exchange and
+// now: airfoil + flap (nf = 800, ~460 steps a solve) 9.38 -> 6.55; plate (nf =
+// 202) 6.74 -> 4.83; flexible plate 6.69 -> 4.82; GMRES(30) of the cylinder
+// (nf = 314) 5.99 -> 3.56; a 42-entry system 5.77 -> 4.15.
 // ------------------------------------------------------------------------
 constexpr int kCwBlk = 32;
+constexpr int kCwLd = kCwBlk + 1;  // row stride of a staged block (no bank conflicts down a column)
+constexpr unsigned long long kUnset = 0x7ff4c0de5eed0001ull;
 
 struct GmCoopWArgs {
-  int nf, kmax, maxit, P, R, NL;
+  int nf, kmax, maxit, P, lPg, R, NL;  // Pg = 2^lPg: the power of two >= P
   int xcd;  // the XCD whose workgroups take part (-1: workgroups 0, 8, 16, ...)
   int l2x;  // 1: exchange through one XCD's L2 when every workgroup is found there
   const double* S;
@@ -1279,13 +858,14 @@ struct GmCoopWArgs {
   GmresDev* s;
   double rtol, atol;
   unsigned* sync;  // [0] error, [8 + c] barriers passed by workgroup c
-  double* dots;    // P x (kmax + 2) partial CGS coefficients
-  double* norms;   // P x 4 partial squared norms
-  double* wfull;   // nf: w (or r) rows of every workgroup
-  double* Hg;      // kmax x (kmax + 1): the rotated Hessenberg, column it at Hg + it (kmax + 1)
+  double* x1;      // 3 x (kmax + 1) x Pg: partial CGS coefficients, coefficient j of workgroup q at j Pg + q
+  double* x2;      // 3 x (kmax + 1): summed CGS coefficients
+  double* x3;      // 3 x nf: the new vector, unnormalised
+  double* rfull;   // nf: the residual at a cycle's start
+  double* norms;   // P x 2: partial squared norms of r and b
   double* yg;      // kmax + 1: the back substitution's y
-  double* hg;      // kmax + 1: the summed CGS coefficients of the step
-  double* Rd;      // kmax + 1: diagonal of the rotated Hessenberg matrix
+  double* Ht;      // (kmax + 1) x kmax: the Hessenberg matrix, entry (j, k) at j kmax + k
+  double* rot;     // 3 kmax: the rotations and the rotated diagonal, (c_k, s_k, d_k) at 3k
   double* Vg;      // P x R x (kmax + 1 - NL): basis vectors NL.. of each workgroup's rows
 };
 
@@ -1302,53 +882,90 @@ __device__ __forceinline__ double gw_reduce2(double v0, double v1) {
   k += gm_dpp<0x4E>(k);
   k += gm_dpp<0x124>(k);
   k += gm_dpp<0x128>(k);
-  k += __shfl_xor(k, 16);
-  k += __shfl_xor(k, 32);
-  return k;
+  return gm_add_xor32(gm_add_xor16(k));
+}
+// the same for RW = 2 or 4 rows; lane l < RW gets the sum of row gw_row<RW>(l)
+template <int RW>
+__device__ __forceinline__ double gw_reduce_rows(const double (&v)[RW]) {
+  if constexpr (RW == 2) return gw_reduce2(v[0], v[1]);
+  else return gc_reduce4(v[0], v[1], v[2], v[3]);
+}
+template <int RW>
+__device__ __forceinline__ int gw_row(int l) {
+  if constexpr (RW == 2) return l & 1;
+  else return ((l & 1) << 1) | ((l >> 1) & 1);
 }
 
 // Butterfly sum over aligned groups of g = 1, 2, 4, ..., 32 consecutive
-// lanes (xor 1 and xor 2 through DPP, xor 4, 8, 16 through lane shuffles):
-// every lane of a group ends with the same bits, ((p0 + p1) + (p2 + p3)) +
-// ... in one fixed order.  The whole wavefront must be active.
+// lanes: xor 1 and xor 2 through DPP quad permutes; then, since all lanes of a
+// quad (of 8 lanes) hold the same bits, xor 4 (8) as a mirror of 8 (16)
+// lanes, and xor 16 by swapping rows.  Every lane of a group ends with the
+// same bits, ((p0 + p1) + (p2 + p3)) + ... in one fixed order.  The whole
+// wavefront must be active.
 __device__ __forceinline__ double gw_group_sum(double p, int g) {
   if (g >= 2) p += gm_dpp<0xB1>(p);
   if (g >= 4) p += gm_dpp<0x4E>(p);
-  if (g >= 8) p += __shfl_xor(p, 4);
-  if (g >= 16) p += __shfl_xor(p, 8);
-  if (g >= 32) p += __shfl_xor(p, 16);
+  if (g >= 8) p += gm_dpp<0x141>(p);
+  if (g >= 16) p += gm_dpp<0x140>(p);
+  if (g >= 32) p = gm_add_xor16(p);
   return p;
 }
 
-// Lanes per CGS coefficient in the dot phase of step it: as many
-// as the 1024 threads allow, up to 8 (groups never straddle a wavefront).
-__device__ __forceinline__ int gw_lanes_per_coef(int it) {
+// Lanes per CGS coefficient in the dot phase of step it (its logarithm): as
+// many as the 1024 threads allow, up to 8 (groups never straddle a wavefront).
+__device__ __forceinline__ int gw_log_lanes_per_coef(int it) {
   const int n = it + 1;
-  return 8 * n <= kGmT ? 8 : (4 * n <= kGmT ? 4 : (2 * n <= kGmT ? 2 : 1));
+  return 8 * n <= kGmT ? 3 : (4 * n <= kGmT ? 2 : (2 * n <= kGmT ? 1 : 0));
 }
 
-// Wavefront-wide sum of p[q * stride] over q < P (lane q loads one value,
-// one memory round trip; fixed reduction order, so every workgroup that
-// runs it gets the same bits).
+// gm_block_sum2 without its 16 loads in flight (they would cost the solve the
+// registers that hold S)
+__device__ __forceinline__ double gw_block_sum(double v, double* red) {
+  const int t = gm_opaque(threadIdx.x);
+  v = gm_wave_sum(v);
+  if ((t & 63) == 0) red[t >> 6] = v;
+  __syncthreads();
+  double tot = 0.0;
+#pragma unroll 1
+  for (int q = 0; q < kGmT / 64; ++q) tot += red[q];
+  __syncthreads();
+  return tot;
+}
+
+// a product rounded by itself, whatever it is added to
+__device__ __forceinline__ double gw_mul(double a, double b) {
+#pragma clang fp contract(off)
+  return a * b;
+}
 
 // Exchange between the workgroups of a cooperative solve.  Loads are
 // device-scope atomic loads: they bypass the CU's L1 and are served by L2
 // (measured on MI355X: ~90 ns per dependent load, against ~56 ns for an L1
-// hit).  Stores: device scope, coherent across XCDs, or with X2 (every
-// workgroup on one XCD, checked at the start of the launch) workgroup-scope
-// stores, which complete at that XCD's L2 -- the one L2 every load of the
-// exchange reads -- instead of at memory.  Each wavefront waits for its
-// stores to complete before a barrier either way.
-template <bool X2>
+// hit); an atomic load is always a vector memory access, where a plain load
+// of a uniform address could be served by the scalar cache.  Stores: device
+// scope, coherent across XCDs, or with X2 (every workgroup on one XCD, checked
+// at the start of the launch) workgroup-scope stores, which complete at that
+// XCD's L2 -- the one L2 every load of the exchange reads -- instead of at
+// memory.
 __device__ __forceinline__ double xc_ld(const double* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 template <bool X2>
-__device__ __forceinline__ void xc_st(double* p, double v) {
-  if constexpr (X2) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-  else __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+__device__ __forceinline__ void xc_st_bits(double* p, unsigned long long v) {
+  unsigned long long* q = reinterpret_cast<unsigned long long*>(p);
+  if constexpr (X2) __hip_atomic_store(q, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  else __hip_atomic_store(q, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 template <bool X2>
+__device__ __forceinline__ void xc_st(double* p, double v) {
+  xc_st_bits<X2>(p, (unsigned long long)__double_as_longlong(v));
+}
+// publishes a value that others poll; any NaN becomes the quiet one, so that
+// it is never taken for kUnset
+template <bool X2>
+__device__ __forceinline__ void xc_put(double* p, double v) {
+  xc_st_bits<X2>(p, v == v ? (unsigned long long)__double_as_longlong(v) : 0x7ff8000000000000ull);
+}
 __device__ __forceinline__ unsigned xc_ldu(const unsigned* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -1357,8 +974,59 @@ __device__ __forceinline__ void xc_stu(unsigned* p, unsigned v) {
   if constexpr (X2) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   else __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// Grid barrier number k over the P workgroups, as gc_sync, with the
-// exchange stores of X2.
+
+// Whether a wavefront that has polled n times gives up: after kCoopSpin polls,
+// or when another wavefront or workgroup has.  The error words are then set,
+// the wavefront goes on with what it has, and the workgroup leaves at its next
+// check of s_err.
+__device__ __forceinline__ bool xc_give_up(long n, unsigned* err, int* s_err) {
+  if ((n & 63) != 0 || (n <= kCoopSpin && xc_ldu(err) == 0u && *(volatile int*)s_err == 0)) return false;
+  if ((threadIdx.x & 63) == 0) {
+    __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    *(volatile int*)s_err = 1;
+  }
+  return true;
+}
+
+// The published value at p for the lanes that need one (0 for the others):
+// the wavefront polls until all of them are there.  The whole wavefront must
+// be active.
+__device__ __forceinline__ double xc_poll(const double* p, bool need, unsigned* err, int* s_err) {
+  unsigned long long v = 0;
+  long n = 0;
+  while (true) {
+    if (need)
+      v = __hip_atomic_load(reinterpret_cast<const unsigned long long*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (__all(!need || v != kUnset)) break;
+    if (xc_give_up(++n, err, s_err)) break;
+  }
+  return __longlong_as_double((long long)v);
+}
+
+// Two published values, polled together.
+__device__ __forceinline__ double2 xc_poll2(const double* p0, bool need0, const double* p1, bool need1, unsigned* err,
+                                            int* s_err) {
+  unsigned long long v0 = 0, v1 = 0;
+  long n = 0;
+  while (true) {
+    if (need0)
+      v0 = __hip_atomic_load(reinterpret_cast<const unsigned long long*>(p0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (need1)
+      v1 = __hip_atomic_load(reinterpret_cast<const unsigned long long*>(p1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (__all((!need0 || v0 != kUnset) && (!need1 || v1 != kUnset))) break;
+    if (xc_give_up(++n, err, s_err)) break;
+  }
+  return make_double2(__longlong_as_double((long long)v0), __longlong_as_double((long long)v1));
+}
+
+// Grid barrier number k (1, 2, ...) over the P workgroups, for the few
+// exchanges outside the Arnoldi steps.  Every wavefront waits for its own
+// stores to complete (gc_wait_stores) before the workgroup barrier, so when
+// wavefront 0 then publishes flag[c] = k every store of workgroup c is
+// visible to the others' loads; wavefront 0 polls the P flags (one lane each)
+// until all have reached k, and the others wait at the second workgroup
+// barrier.  Bounded: on a timeout (or another workgroup's) the error word is
+// set and every workgroup leaves.
 template <bool X2>
 __device__ __forceinline__ bool xc_sync(unsigned* sync, int P, int c, unsigned k, int* s_err) {
   gc_wait_stores();
@@ -1371,11 +1039,11 @@ __device__ __forceinline__ bool xc_sync(unsigned* sync, int P, int c, unsigned k
     if (lane == 0) xc_stu<X2>(fl + c, k);
     long n = 0;
     while (true) {
-      const unsigned v = lane < P ? xc_ldu<X2>(fl + lane) : k;
+      const unsigned v = lane < P ? xc_ldu(fl + lane) : k;
       if (__all(v >= k)) break;
-      if (xc_ldu<X2>(err) != 0u || ++n > kCoopSpin) {
+      if (xc_ldu(err) != 0u || ++n > kCoopSpin) {
         if (lane == 0) {
-          xc_stu<X2>(err, 1u);
+          __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           *s_err = 1;
         }
         break;
@@ -1388,141 +1056,132 @@ __device__ __forceinline__ bool xc_sync(unsigned* sync, int P, int c, unsigned k
   return *s_err == 0;
 }
 
-// Block-wide sums of two values (every thread gets both), in a fixed order:
-// each wavefront's sum (gm_wave_sum), then the 16 wavefront sums by a row of
-// 16 lanes (gm_row_sum16).  red holds at least 2 kGmT / 64 doubles; it is
-// read after the one workgroup barrier here, so the caller must pass another
-// barrier before red is written again.
-__device__ __forceinline__ void gw_block_sum_pair(double& a, double& b, double* red) {
-  const int t = gm_opaque(threadIdx.x), l = t & 63;
-  a = gm_wave_sum(a);
-  b = gm_wave_sum(b);
-  if (l == 0) {
-    red[t >> 6] = a;
-    red[kGmT / 64 + (t >> 6)] = b;
-  }
-  __syncthreads();
-  // lanes 0..15 of every wavefront take the 16 partials of a, lanes 16..31
-  // those of b: one LDS read per lane, then a sum over each row of 16 lanes
-  double v = l < 2 * (kGmT / 64) ? red[l] : 0.0;
-  v = gm_row_sum16(v);
-  a = gm_readlane(v, 0);
-  b = gm_readlane(v, 16);
-}
-
+// Sets what workgroup c published in a step of n coefficients to kUnset, in
+// copy k of the buffers (threads t, t + nthr, ...).
 template <bool X2>
-__device__ __forceinline__ double gw_wave_gather(const double* p, long stride, int P, int lane) {
-  const double v = lane < P ? xc_ld<X2>(p + (long)lane * stride) : 0.0;
-  return gm_wave_sum(v);
+__device__ __forceinline__ void coopw_clear(const GmCoopWArgs& a, int c, int r0, int Rc, int k, int n, int t, int nthr) {
+  double* x1 = a.x1 + ((k * (a.kmax + 1)) << a.lPg) + c;
+  double* x2 = a.x2 + k * (a.kmax + 1);
+  for (int j = t; j < n; j += nthr) xc_st_bits<X2>(x1 + (j << a.lPg), kUnset);
+  for (int j = c + t * a.P; j < n; j += nthr * a.P) xc_st_bits<X2>(x2 + j, kUnset);
+  for (int r = t; r < Rc; r += nthr) xc_st_bits<X2>(a.x3 + k * a.nf + r0 + r, kUnset);
 }
 
-template <int CQ, bool X2>
+template <int RW, int CQ, bool X2>
 __device__ __forceinline__ void coopw_solve(const GmCoopWArgs& a, int c, unsigned bk, double* dyn, double* red,
                                             double* s_val, int* s_flag, int* s_err) {
-  const int nf = a.nf, kmax = a.kmax, ld = kmax + 1, T = kGmT, R = a.R, NL = a.NL;
-  const int r0 = c * R, Rc = max(0, min(nf, r0 + R) - r0);
+  constexpr int kLast = kGmT / 64 - 1;
+  const int nf = a.nf, kmax = a.kmax, ld = kmax + 1, T = kGmT, R = a.R, NL = a.NL, P = a.P, lPg = a.lPg, Pg = 1 << lPg;
+  const int r0 = c * R, Rc = min(nf, r0 + R) - r0;
   const int ldg = ld - NL;  // row stride of the basis vectors kept in HBM
   double* Vgc = a.Vg + (size_t)c * R * (size_t)max(ldg, 0);
-  double* wl = dyn;                    // 32: local rows of w
-  double* hcol = wl + 32;              // kmax + 2: CGS coefficients (y at a cycle's end)
+  double* wl = dyn;                    // 64: local rows of S u
+  double* nrm = wl + 64;               // 32: the workgroups' shares of |u|^2
+  double* hcol = nrm + 32;             // kmax + 2: CGS coefficients of S u (y at a cycle's end)
   double* alpha = hcol + kmax + 2;     // kmax + 2: entry it of the rotated column = sum_j alpha_j h_j
-  double* lcc = alpha + kmax + 2;      // kmax
-  double* lss = lcc + kmax;            // kmax
-  double* grs = lss + kmax;            // kmax + 1 (y of the back substitution in place)
-  double* stg = grs + kmax + 1;        // kCwBlk^2: a diagonal block of the back substitution
-  double* ub = stg + kCwBlk * kCwBlk;  // nf: the vector of a product, copied once from L2
+  double* grs = alpha + kmax + 2;      // kmax + 1 (y of the back substitution in place)
+  double* stg = grs + kmax + 1;        // kCwBlk x kCwLd: a diagonal block of the back substitution
+  double* ub = stg + kCwBlk * kCwLd;   // nf: the vector of a product, u
   double* Vl = ub + nf;                // R NL: local rows of basis vectors 0..NL-1, row-major
-  // rows 2 wq and 2 wq + 1 of S, columns ln + 64 k, in registers (0 outside the matrix)
-  double s0[CQ], s1[CQ];
+  // rows RW wq .. of S, columns ln + 64 k, in registers (0 outside the matrix)
+  double s[RW][CQ];
   {
     const int wq = threadIdx.x >> 6, ln = threadIdx.x & 63;
-    const int ra = 2 * wq, rb = 2 * wq + 1;
 #pragma unroll
-    for (int k = 0; k < CQ; ++k) {
-      const int col = ln + 64 * k;
-      s0[k] = ra < Rc && col < nf ? a.S[(long)col * nf + r0 + ra] : 0.0;
-      s1[k] = rb < Rc && col < nf ? a.S[(long)col * nf + r0 + rb] : 0.0;
-    }
+    for (int i = 0; i < RW; ++i)
+#pragma unroll
+      for (int k = 0; k < CQ; ++k) {
+        const int row = RW * wq + i, col = ln + 64 * k;
+        s[i][k] = row < Rc && col < nf ? a.S[(long)col * nf + r0 + row] : 0.0;
+      }
   }
   __syncthreads();
 
-  // S[local rows] u for a vector u the workgroups left in L2: the
-  // workgroup copies u into LDS once (ub; one load per thread), then every
-  // lane reads the CQ entries it multiplies from there, so the L2 serves u
-  // once per workgroup instead of once per wavefront.  Lanes 0 and 1 of
-  // wavefront q get rows 2q and 2q + 1 (0 in the other lanes).  Every
-  // thread must call it (a workgroup barrier follows the copy); ub is next
-  // written by the following call, after at least one more barrier.
-  auto matvec_g = [&](const double* u) -> double {
-    for (int i = gm_opaque(threadIdx.x); i < nf; i += T) ub[i] = xc_ld<X2>(u + i);
-    __syncthreads();
+  // wl = S[local rows] ub (wavefront q: rows RW q ..)
+  auto matvec = [&]() {
     const int q = gm_opaque(threadIdx.x) >> 6, l = gm_opaque(threadIdx.x) & 63;
-    double sum = 0.0;
-    if (2 * q < Rc) {  // uniform over the wavefront
-      double v[CQ];
+    if (RW * q < Rc) {  // uniform over the wavefront
+      double v[CQ], acc[RW];
 #pragma unroll
       for (int k = 0; k < CQ; ++k) v[k] = ub[min(l + 64 * k, nf - 1)];
-      double acc0 = 0.0, acc1 = 0.0;
 #pragma unroll
-      for (int k = 0; k < CQ; ++k) {
-        acc0 += s0[k] * v[k];  // s0, s1 are 0 past the matrix
-        acc1 += s1[k] * v[k];
+      for (int i = 0; i < RW; ++i) {
+        acc[i] = 0.0;
+#pragma unroll
+        for (int k = 0; k < CQ; ++k) acc[i] += s[i][k] * v[k];  // s is 0 past the matrix
       }
-      sum = gw_reduce2(acc0, acc1);
+      const double sum = gw_reduce_rows<RW>(acc);
+      const int row = RW * q + gw_row<RW>(l);
+      if (l < RW && row < Rc) wl[row] = sum;
     }
-    return sum;
   };
-  // lanes 0/1 of the row-pair wavefronts store their row of S u times scale
-  auto store_rows = [&](double sum, double scale) {
-    const int q = gm_opaque(threadIdx.x) >> 6, l = gm_opaque(threadIdx.x) & 63;
-    const int row = 2 * q + (l & 1);
-    if (2 * q < Rc && l < 2 && row < Rc) wl[row] = sum * scale;
-  };
-  // acc0/acc1 += sum_{j = l, l + 64, ... < jn} coef[j] V(ra / rb, j)
-  auto rowpair = [&](const double* coef, int jn, int ra, int rb, int l, double& acc0, double& acc1) {
-    const int ja = min(jn, NL);
-    int j = l;
-#pragma unroll 8
-    for (; j < ja; j += 64) {
+  // acc[i] += sum_{j = l, l + 64, ... < jn} coef[j] V(RW q + i, j): four
+  // chunks of 64 vectors in flight while all are in LDS (terms past jn add 0)
+  auto rows_dot = [&](const double* coef, int jn, int q, int l, double (&acc)[RW]) {
+    int rr[RW];
+#pragma unroll
+    for (int i = 0; i < RW; ++i) rr[i] = min(RW * q + i, Rc - 1) * NL;
+    if (jn <= NL) {
+#pragma unroll 1
+      for (int w = 0; w < jn; w += 256) {
+        double h[4], v[4][RW];
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+          const int j = min(w + 64 * b + l, jn - 1);
+          h[b] = coef[j];
+#pragma unroll
+          for (int i = 0; i < RW; ++i) v[b][i] = Vl[rr[i] + j];
+        }
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+          for (int i = 0; i < RW; ++i) acc[i] += (w + 64 * b + l < jn ? h[b] : 0.0) * v[b][i];
+      }
+      return;
+    }
+#pragma unroll 1
+    for (int j = l; j < jn; j += 64) {
       const double h = coef[j];
-      acc0 += h * Vl[ra * NL + j];
-      acc1 += h * Vl[rb * NL + j];
-    }
-    for (; j < jn; j += 64) {
-      const double h = coef[j];
-      acc0 += h * Vgc[(size_t)ra * ldg + (j - NL)];
-      acc1 += h * Vgc[(size_t)rb * ldg + (j - NL)];
+#pragma unroll
+      for (int i = 0; i < RW; ++i)
+        acc[i] += h * (j < NL ? Vl[rr[i] + j] : Vgc[(size_t)min(RW * q + i, Rc - 1) * ldg + (j - NL)]);
     }
   };
+
   int its = 0, reason = 0, first = 1;
   double rn0 = 0.0, ttol = 0.0;
+  bool ok = true;
   while (true) {
     // ---- cycle start: r = b - S x (x from every workgroup's rows)
-    store_rows(matvec_g(a.x), 1.0);
+    for (int i = gm_opaque(threadIdx.x); i < nf; i += T) ub[i] = xc_ld(a.x + i);
+    __syncthreads();
+    matvec();
     __syncthreads();
     double pr = 0.0, pb = 0.0;
     for (int r = gm_opaque(threadIdx.x); r < Rc; r += T) {
       const double bv = a.b[r0 + r];
       const double rv = bv - wl[r];
-      xc_st<X2>(a.wfull + r0 + r, rv);
+      xc_st<X2>(a.rfull + r0 + r, rv);
       pr += rv * rv;
       pb += bv * bv;
     }
-    pr = gm_block_sum2(pr, red, T);
-    pb = gm_block_sum2(pb, red, T);
+    pr = gw_block_sum(pr, red);
+    pb = gw_block_sum(pb, red);
     if (threadIdx.x == 0) {
-      xc_st<X2>(a.norms + c * 4 + 1, pr);
-      xc_st<X2>(a.norms + c * 4 + 2, pb);
+      xc_st<X2>(a.norms + c * 2, pr);
+      xc_st<X2>(a.norms + c * 2 + 1, pb);
     }
-    if (!xc_sync<X2>(a.sync, a.P, c, ++bk, s_err)) break;
+    if (!xc_sync<X2>(a.sync, P, c, ++bk, s_err)) break;
     if (threadIdx.x < 64) {
-      const double sr = gw_wave_gather<X2>(a.norms + 1, 4, a.P, threadIdx.x);
-      const double sb = gw_wave_gather<X2>(a.norms + 2, 4, a.P, threadIdx.x);
-      if (threadIdx.x == 0) {
+      const int lane = threadIdx.x;
+      const double sr = gm_wave_sum(lane < P ? xc_ld(a.norms + lane * 2) : 0.0);
+      const double sb = gm_wave_sum(lane < P ? xc_ld(a.norms + lane * 2 + 1) : 0.0);
+      if (lane == 0) {
         s_val[0] = sr;
         s_val[1] = sb;
       }
     }
+    for (int i = gm_opaque(threadIdx.x); i < nf; i += T) ub[i] = xc_ld(a.rfull + i);
     __syncthreads();
     const double res0 = sqrt(s_val[0]), bn = sqrt(s_val[1]);
     if (first) {
@@ -1533,226 +1192,314 @@ __device__ __forceinline__ void coopw_solve(const GmCoopWArgs& a, int c, unsigne
     if (res0 == 0.0 || res0 <= ttol) reason = 1;
     else if (res0 >= 1e4 * rn0) reason = -1;
     if (reason) break;
-    if (threadIdx.x == 0) {
-      grs[0] = res0;
-      alpha[0] = 1.0;
-    }
-    // v_0 = r / res0 and w = S v_0 (the row sums of S r scaled by 1 / res0)
-    const double inv0 = 1.0 / res0;
-    store_rows(matvec_g(a.wfull), inv0);
-    for (int r = gm_opaque(threadIdx.x); r < Rc; r += T) {
-      const double v = xc_ld<X2>(a.wfull + r0 + r) * inv0;
-      if (NL > 0) Vl[r * NL] = v;
-      else Vgc[(size_t)r * ldg] = v;
-    }
-    __syncthreads();
-    int it = 0;
-    bool ok = true;
+    __syncthreads();  // s_val is rewritten below
+    int it = 0;         // columns formed
+    int cur = 0, old = 2;  // it mod 3, (it - 1) mod 3
+    double hv = 0.0;    // last wavefront: entry it - 1 of column it - 1 after the previous rotations
+    double cc = 1.0, sn = 0.0;  // last wavefront: the rotation of column it - 1
     while (true) {
-      // here wl = S v_it on the local rows
-      // partial CGS coefficient <w, v_j> over the local rows: g lanes per
-      // j, lane sub takes rows sub, sub + g, ...
-      const int g = gw_lanes_per_coef(it);
-      {
-        const int t = gm_opaque(threadIdx.x), j = t / g, sub = t - j * g;
-        double p = 0.0;
-        if (j <= it) {
-          if (j < NL) {
-#pragma unroll 8
-            for (int r = sub; r < Rc; r += g) p += wl[r] * Vl[r * NL + j];
-          } else {
-            const double* vg = Vgc + (j - NL);
-#pragma unroll 8
-            for (int r = sub; r < Rc; r += g) p += wl[r] * vg[(size_t)r * ldg];
-          }
-        }
-        p = gw_group_sum(p, g);
-        if (j <= it && sub == 0) xc_st<X2>(a.dots + (long)c * (kmax + 2) + j, p);
+      // here ub = u, the unnormalised vector v_it
+      const bool more = it < kmax && its < a.maxit;
+      double tt = res0;  // last wavefront: |u|
+      matvec();
+      if (gm_opaque(threadIdx.x) >= T - 64) {
+        const int lane = gm_opaque(threadIdx.x) & 63;
+        if (it > 0) tt = sqrt(gm_wave_sum(lane < P ? nrm[lane] : 0.0));
+        if (lane == 0) s_val[0] = 1.0 / tt;
       }
-      if (!xc_sync<X2>(a.sync, a.P, c, ++bk, s_err)) {
-        ok = false;
-        break;
-      }
-      // h_j: workgroup c sums the P partials of j = c, c + P, ... (lane q of
-      // a group of P lanes loads partial q; fixed butterfly over the group)
-      // and publishes it; after a barrier every workgroup loads all h_j.
-      // Each partial is read once, not once per workgroup.
-      {
-        const int t = gm_opaque(threadIdx.x), jj = t / a.P, q = t - jj * a.P;
-        const int j = c + jj * a.P;
-        double h = j <= it ? xc_ld<X2>(a.dots + (long)q * (kmax + 2) + j) : 0.0;
-        h = gw_group_sum(h, a.P);
-        if (j <= it && q == 0) xc_st<X2>(a.hg + j, h);
-      }
-      if (!xc_sync<X2>(a.sync, a.P, c, ++bk, s_err)) {
-        ok = false;
-        break;
-      }
-      for (int j = gm_opaque(threadIdx.x); j <= it; j += T) hcol[j] = xc_ld<X2>(a.hg + j);
+      if (threadIdx.x == 0) s_flag[2] = *(volatile int*)s_err;
       __syncthreads();
-      // w -= sum_j h_j v_j on the local rows; partial ||w||^2; w rows out.
-      // The same block reduction forms sum_j alpha_j h_j, entry it of the
-      // new Hessenberg column after the previous rotations (identical bits
-      // in every workgroup: the same alpha, h and order).
-      double hv;
-      {
-        const int q = gm_opaque(threadIdx.x) >> 6, l = gm_opaque(threadIdx.x) & 63;
-        double pn = 0.0;
-        if (2 * q < Rc) {  // uniform over the wavefront
-          const int ra = 2 * q, rb = 2 * q + 1 < Rc ? 2 * q + 1 : 2 * q;
-          double acc0 = 0.0, acc1 = 0.0;
-          rowpair(hcol, it + 1, ra, rb, l, acc0, acc1);
-          const double sum = gw_reduce2(-acc0, -acc1);
-          const int row = 2 * q + (l & 1);
-          if (l < 2 && row < Rc) {
-            const double wn = wl[row] + sum;
-            wl[row] = wn;
-            xc_st<X2>(a.wfull + r0 + row, wn);
-            pn = wn * wn;
-          }
-        }
-        const int t = gm_opaque(threadIdx.x);
-        double ah = t <= it ? alpha[t] * hcol[t] : 0.0;  // it < kGmT
-        gw_block_sum_pair(pn, ah, red);
-        hv = ah;
-        if (threadIdx.x == 0) xc_st<X2>(a.norms + c * 4, pn);
-      }
-      if (!xc_sync<X2>(a.sync, a.P, c, ++bk, s_err)) {
+      if (s_flag[2]) {
         ok = false;
         break;
       }
-      // this thread's local-row entry of the new vector w (unnormalised),
-      // the row sums of S w for the next step (from L2, beside the norm
-      // partials and the Givens step of wavefront 0)
-      const int t0 = gm_opaque(threadIdx.x);
-      // wavefront 0 loads the P norm partials before the product's vector
-      // (lane q partial q, as gw_wave_gather), so that the two L2 round
-      // trips overlap
-      const double npart = t0 < a.P ? xc_ld<X2>(a.norms + (long)t0 * 4) : 0.0;
-      const double swsum = matvec_g(a.wfull);
-      const double wpre_l = t0 < Rc ? ub[r0 + t0] : 0.0;
-      if (gm_opaque(threadIdx.x) < 64) {
-        const int lane = gm_opaque(threadIdx.x);
-        const double tt = sqrt(gm_wave_sum(npart));
-        if (lane == 0) {
-          // KSPGMRESUpdateHessenberg: tt < min(|tt / grs[it]|, 1e-30) is a
-          // happy breakdown (the quotient is needed only when tt < 1e-30)
-          const int hap = tt < 1e-30 && tt < fabs(tt / grs[it]);
-          double res, diag, cc = 1.0, sn = 0.0;
+      const double inv = s_val[0];  // v_it = u inv, S v_it = (S u) inv
+      // partial CGS coefficients <S v_it, v_j>, j <= it, over the local
+      // rows: g lanes per j, lane sub takes rows sub, sub + g, ...; blocks of
+      // four rows, the loads of a block ahead of its sums (the rows past Rc
+      // add 0)
+      if (more) {
+        const int lg = gw_log_lanes_per_coef(it), g = 1 << lg;
+        const int t = gm_opaque(threadIdx.x), j = t >> lg, sub = t & (g - 1);
+        if (((t & ~63) >> lg) <= it) {  // uniform over the wavefront
+          double p = 0.0;
+          if (j < it && j >= NL) {
+            const double* vg = Vgc + (j - NL);
+#pragma unroll 1
+            for (int r1 = sub; r1 < Rc; r1 += 4 * g) {
+              double w[4], v[4];
+#pragma unroll
+              for (int i = 0; i < 4; ++i) {
+                const int rr = min(r1 + (i << lg), Rc - 1);
+                w[i] = wl[rr];
+                v[i] = vg[(size_t)rr * ldg];
+              }
+#pragma unroll
+              for (int i = 0; i < 4; ++i) p += (r1 + (i << lg) < Rc ? gw_mul(w[i], inv) : 0.0) * v[i];
+            }
+          } else if (j <= it) {
+            const double* vl = j < it ? Vl + j : ub + r0;  // v_it is not stored yet
+            const int ldv = j < it ? NL : 1;
+            const double sc = j < it ? 1.0 : inv;
+#pragma unroll 1
+            for (int r1 = sub; r1 < Rc; r1 += 4 * g) {
+              double w[4], v[4];
+#pragma unroll
+              for (int i = 0; i < 4; ++i) {
+                const int rr = min(r1 + (i << lg), Rc - 1);
+                w[i] = wl[rr];
+                v[i] = vl[rr * ldv];
+              }
+#pragma unroll
+              for (int i = 0; i < 4; ++i)
+                p += (r1 + (i << lg) < Rc ? gw_mul(w[i], inv) : 0.0) * gw_mul(v[i], sc);
+            }
+          }
+          p = gw_group_sum(p, g);
+          if (j <= it && sub == 0) xc_put<X2>(a.x1 + ((cur * ld + j) << lPg) + c, p);
+        }
+      }
+      if (gm_opaque(threadIdx.x) >= T - 64) {
+        // the last wavefront: the Givens step of column k = it - 1
+        // (KSPGMRESUpdateHessenberg)
+        const int lane = gm_opaque(threadIdx.x) & 63;
+        int rs = 0;
+        cc = 1.0;
+        sn = 0.0;
+        if (it == 0) {
+          if (lane == 0) grs[0] = res0;
+        } else {
+          const int k = it - 1;
+          const double gk = grs[k];
+          // tt < min(|tt / grs[k]|, 1e-30) is a happy breakdown (the
+          // quotient is needed only when tt < 1e-30)
+          const bool hap = tt < 1e-30 && tt < fabs(tt / gk);
+          double res = 0.0, diag = hv;
           if (!hap) {
             const double t1 = sqrt(hv * hv + tt * tt);
             cc = hv / t1;
             sn = tt / t1;
-            lcc[it] = cc;
-            lss[it] = sn;
-            grs[it + 1] = -sn * grs[it];
-            grs[it] = cc * grs[it];
             diag = cc * hv + sn * tt;
-            res = fabs(grs[it + 1]);
-          } else {
-            diag = hv;
-            res = 0.0;
+            res = fabs(sn * gk);
           }
-          if (c == 0) a.Rd[it] = diag;
-          int rs = 0;
           if (res <= ttol) rs = 1;
           else if (res >= 1e4 * rn0) rs = -1;
           if (hap && !rs) rs = 1;
-          s_flag[0] = rs;
-          s_flag[1] = hap;
-          s_val[0] = tt;
-          s_val[1] = sn;
-          red[2 * (kGmT / 64)] = cc;
+          if (lane == 0) {
+            if (!hap) {
+              grs[it] = -sn * gk;
+              grs[k] = cc * gk;
+            }
+            if (c == 0) {
+              a.rot[3 * k] = cc;
+              a.rot[3 * k + 1] = sn;
+              a.rot[3 * k + 2] = diag;
+            }
+          }
+        }
+        if (lane == 0) s_flag[0] = rs;
+      }
+      if (more) {
+        const int n = it + 1;
+        const double* x1 = a.x1 + ((cur * ld) << lPg);  // below 2^17
+        if ((n << lPg) <= 2 * T) {
+          // few partials: every workgroup sums all of them (Pg lanes per
+          // coefficient, fixed butterfly)
+          for (int base = 0; base < (n << lPg); base += T) {
+            const int i = base + gm_opaque(threadIdx.x), j = i >> lPg, q = i & (Pg - 1);
+            if (((i & ~63) >> lPg) >= n) break;  // uniform over the wavefront
+            const double h = gw_group_sum(xc_poll(x1 + i, j < n && q < P, a.sync, s_err), Pg);
+            if (j < n && q == 0) hcol[j] = h;
+          }
+        } else {
+          // workgroup c sums coefficients c, c + P, ... in the same way and
+          // publishes the sums; each partial is read once
+          for (int base = 0; c + base * P < n; base += T >> lPg) {
+            const int t = gm_opaque(threadIdx.x), jj = base + (t >> lPg), q = t & (Pg - 1);
+            const int j = c + jj * P;
+            if (c + (base + ((t & ~63) >> lPg)) * P >= n) break;  // uniform over the wavefront
+            const double h = gw_group_sum(xc_poll(x1 + (j << lPg) + q, j < n && q < P, a.sync, s_err), Pg);
+            if (j < n && q == 0) xc_put<X2>(a.x2 + cur * ld + j, h);
+          }
+          const int t = gm_opaque(threadIdx.x);  // n <= kmax + 1 <= T
+          if ((t & ~63) < n) {  // uniform over the wavefront
+            const double h = xc_poll(a.x2 + cur * ld + t, t < n, a.sync, s_err);
+            if (t < n) hcol[t] = h;
+          }
         }
       }
       __syncthreads();
       reason = s_flag[0];
-      const int hap = s_flag[1];
-      // workgroup 0 keeps the unrotated column (rows 0..it, then tt); the
-      // rotations are applied to all columns at the cycle's end
-      if (c == 0) {
-        for (int j = gm_opaque(threadIdx.x); j <= it; j += T) a.Hg[(long)it * ld + j] = hcol[j];
-        if (threadIdx.x == 0) a.Hg[(long)it * ld + it + 1] = s_val[0];
-      }
-      if (!hap) {
-        // v_(it+1) = w / tt, and S v_(it+1) for the next step; alpha for the
-        // next column: every entry times -s_it, then c_it
-        const double inv = 1.0 / s_val[0];
-        store_rows(swsum, inv);
-        if (t0 < Rc) {
-          const int j = it + 1;
-          if (j < NL) Vl[t0 * NL + j] = wpre_l * inv;
-          else Vgc[(size_t)t0 * ldg + (j - NL)] = wpre_l * inv;
+      if (reason || !more) break;
+      // the new vector's local rows, S v_it - sum_j h_j v_j
+      {
+        const int q = gm_opaque(threadIdx.x) >> 6, l = gm_opaque(threadIdx.x) & 63;
+        if (RW * q < Rc) {  // uniform over the wavefront
+          double acc[RW];
+#pragma unroll
+          for (int i = 0; i < RW; ++i) acc[i] = 0.0;
+          rows_dot(hcol, it, q, l, acc);
+          if (l == (it & 63)) {  // the term of v_it, the last of its lane
+            const double h = hcol[it];
+#pragma unroll
+            for (int i = 0; i < RW; ++i) acc[i] += h * gw_mul(ub[r0 + min(RW * q + i, Rc - 1)], inv);
+          }
+#pragma unroll
+          for (int i = 0; i < RW; ++i) acc[i] = -acc[i];
+          const double sum = gw_reduce_rows<RW>(acc);
+          gc_wait_stores();  // the clears of the step before
+          const int row = RW * q + gw_row<RW>(l);
+          if (l < RW && row < Rc) {
+            const double v = gw_mul(ub[r0 + row], inv);
+            xc_put<X2>(a.x3 + cur * nf + r0 + row, gw_mul(wl[row], inv) + sum);
+            if (it < NL) Vl[row * NL + it] = v;
+            else Vgc[(size_t)row * ldg + (it - NL)] = v;
+          }
+          // what step it - 1 published
+          if (it > 0)
+            coopw_clear<X2>(a, c, r0, Rc, old, it, gm_opaque(threadIdx.x), 64 * ((Rc + RW - 1) / RW));
         }
-        const double sn = s_val[1];
-        for (int j = gm_opaque(threadIdx.x); j <= it; j += T) alpha[j] = -sn * alpha[j];
-        if (threadIdx.x == 0) alpha[it + 1] = red[2 * (kGmT / 64)];
+      }
+      if (gm_opaque(threadIdx.x) >= T - 64) {
+        const int lane = gm_opaque(threadIdx.x) & 63;
+        double part = 0.0;  // lane w: the sum over j = 64 w ..
+#pragma unroll 1
+        for (int w0 = 0; 64 * w0 <= it; w0 += 4) {
+          double p[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int j = 64 * (w0 + i) + lane, jj = min(j, it);
+            double al = alpha[jj];
+            const double h = hcol[jj];
+            al = j < it ? -sn * al : cc;
+            if (j <= it) alpha[j] = al;
+            p[i] = j <= it ? gw_mul(al, h) : 0.0;
+          }
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const double q = gm_wave_sum(p[i]);
+            if (lane == w0 + i) part = q;
+          }
+        }
+        hv = gm_readlane(gm_row_sum16(part), 0);
+      }
+      if (c == 0) {
+        for (int j = gm_opaque(threadIdx.x); j <= it; j += T) a.Ht[(long)j * kmax + it] = hcol[j];
       }
       ++it;
       ++its;
+      old = cur;
+      cur = cur == 2 ? 0 : cur + 1;
+      // the new vector, two adjacent rows of a workgroup per lane (16 lanes a
+      // workgroup), and the workgroups' shares of its squared norm: the
+      // squares of adjacent rows, then gm_row_sum16
+      {
+        const int t = gm_opaque(threadIdx.x), cq = t >> 4;
+        if ((t >> 6) * 4 < P) {  // uniform over the wavefront
+          const int rend = cq < P ? min(cq * R + R, nf) : 0;
+          double tot = 0.0;
+#pragma unroll
+          for (int b = 0; b < RW / 2; ++b) {
+            const int ra = cq * R + 32 * b + 2 * (t & 15);
+            const bool n0 = ra < rend, n1 = ra + 1 < rend;
+            const double* p = a.x3 + old * nf + ra;
+            const double2 u = xc_poll2(p, n0, p + 1, n1, a.sync, s_err);
+            if (n0) ub[ra] = u.x;
+            if (n1) ub[ra + 1] = u.y;
+            tot += gm_row_sum16(gw_mul(u.x, u.x) + gw_mul(u.y, u.y));
+          }
+          if ((t & 15) == 0 && cq < P) nrm[cq] = tot;
+        }
+      }
       __syncthreads();
-      if (reason || it >= kmax || its >= a.maxit) break;
     }
     if (!ok) break;
-    // ---- KSPGMRESBuildSoln: workgroup 0 solves the rotated triangular
-    // system (grs becomes y in place) and publishes y
+    // ---- KSPGMRESBuildSoln: workgroup 0 rotates the columns, solves the
+    // triangular system (grs becomes y in place) and publishes y
     const int top = it - 1;
     if (c == 0) {
-      // the previous rotations on every column k (thread k; the same
-      // recurrence as KSPGMRESUpdateHessenberg), its diagonal from the step
+      double* rc = hcol;   // the rotations (hcol and alpha are free here)
+      double* rsn = alpha;
       for (int k = gm_opaque(threadIdx.x); k <= top; k += T) {
-        double* col = a.Hg + (long)k * ld;
+        rc[k] = a.rot[3 * k];
+        rsn[k] = a.rot[3 * k + 1];
+      }
+      __syncthreads();
+      // the previous rotations on every column k (thread k), its diagonal
+      // from the step: the rows are read across the columns, eight rows
+      // ahead of the recurrence
+      for (int k = gm_opaque(threadIdx.x); k <= top; k += T) {
+        double* col = a.Ht + k;
         double carry = col[0];
-        for (int j = 0; j < k; ++j) {
-          const double hn = col[j + 1];
-          col[j] = lcc[j] * carry + lss[j] * hn;
-          carry = -lss[j] * carry + lcc[j] * hn;
+        for (int j0 = 0; j0 < k; j0 += 8) {
+          double h[8];
+#pragma unroll
+          for (int i = 0; i < 8; ++i) h[i] = col[(long)min(j0 + i + 1, k) * kmax];
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            const int j = j0 + i;
+            if (j < k) {
+              const double hn = h[i];
+              col[(long)j * kmax] = rc[j] * carry + rsn[j] * hn;
+              carry = -rsn[j] * carry + rc[j] * hn;
+            }
+          }
         }
-        col[k] = a.Rd[k];
+        col[(long)k * kmax] = a.rot[3 * k + 2];
       }
       __syncthreads();
       for (int kb1 = top; kb1 >= 0; kb1 -= kCwBlk) {
         const int kb0 = max(0, kb1 - kCwBlk + 1), nb = kb1 - kb0 + 1;
-        // column k of the diagonal block: stg[k kCwBlk + i] = H(kb0 + i, kb0 + k), i <= k
-        for (int q = gm_opaque(threadIdx.x); q < nb * nb; q += T) {
-          const int k = q / nb, i = q - k * nb;
-          if (i <= k) stg[k * kCwBlk + i] = a.Hg[(long)(kb0 + k) * ld + kb0 + i];
+        // row i, column k of the diagonal block at i kCwLd + k
+        {
+          const int i = gm_opaque(threadIdx.x) / kCwBlk, k = gm_opaque(threadIdx.x) % kCwBlk;
+          if (k < nb && i <= k) stg[i * kCwLd + k] = a.Ht[(long)(kb0 + i) * kmax + kb0 + k];
         }
         __syncthreads();
         if (threadIdx.x < 64) {
           const int lane = threadIdx.x;
           double ti = lane < nb ? grs[kb0 + lane] : 0.0;
           for (int k = nb - 1; k >= 0; --k) {
-            const double yk = gm_readlane(ti, k) / stg[k * kCwBlk + k];
-            if (lane < k) ti -= stg[k * kCwBlk + lane] * yk;
+            const double yk = gm_readlane(ti, k) / stg[k * kCwLd + k];
+            if (lane < k) ti -= stg[lane * kCwLd + k] * yk;
             if (lane == k) ti = yk;
           }
           if (lane < nb) grs[kb0 + lane] = ti;
         }
         __syncthreads();
-        // the rows above the block, columns of the block in descending order
+        // the rows above the block, columns of the block in descending
+        // order, eight loads ahead
         for (int i = gm_opaque(threadIdx.x); i < kb0; i += T) {
+          const double* row = a.Ht + (long)i * kmax + kb0;
           double t = grs[i];
-          for (int k = nb - 1; k >= 0; --k) t -= a.Hg[(long)(kb0 + k) * ld + i] * grs[kb0 + k];
+          for (int k0 = nb - 1; k0 >= 0; k0 -= 8) {
+            double h[8];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) h[q] = row[max(k0 - q, 0)];
+#pragma unroll
+            for (int q = 0; q < 8; ++q)
+              if (k0 - q >= 0) t -= h[q] * grs[kb0 + k0 - q];
+          }
           grs[i] = t;
         }
         __syncthreads();
       }
       for (int j = gm_opaque(threadIdx.x); j <= top; j += T) xc_st<X2>(a.yg + j, grs[j]);
     }
-    if (!xc_sync<X2>(a.sync, a.P, c, ++bk, s_err)) break;
-    for (int j = gm_opaque(threadIdx.x); j <= top; j += T) hcol[j] = xc_ld<X2>(a.yg + j);
+    if (!xc_sync<X2>(a.sync, P, c, ++bk, s_err)) break;
+    for (int j = gm_opaque(threadIdx.x); j <= top; j += T) hcol[j] = xc_ld(a.yg + j);
     __syncthreads();
     // x += V y on the local rows
     {
       const int q = gm_opaque(threadIdx.x) >> 6, l = gm_opaque(threadIdx.x) & 63;
-      if (2 * q < Rc) {
-        const int ra = 2 * q, rb = 2 * q + 1 < Rc ? 2 * q + 1 : 2 * q;
-        double acc0 = 0.0, acc1 = 0.0;
-        rowpair(hcol, top + 1, ra, rb, l, acc0, acc1);
-        const double sum = gw_reduce2(acc0, acc1);
-        const int row = 2 * q + (l & 1);
-        if (l < 2 && row < Rc) xc_st<X2>(a.x + r0 + row, xc_ld<X2>(a.x + r0 + row) + sum);
+      if (RW * q < Rc) {
+        double acc[RW];
+#pragma unroll
+        for (int i = 0; i < RW; ++i) acc[i] = 0.0;
+        rows_dot(hcol, top + 1, q, l, acc);
+        const double sum = gw_reduce_rows<RW>(acc);
+        const int row = RW * q + gw_row<RW>(l);
+        if (l < RW && row < Rc) xc_st<X2>(a.x + r0 + row, xc_ld(a.x + r0 + row) + sum);
       }
     }
     if (reason) break;
@@ -1760,7 +1507,11 @@ __device__ __forceinline__ void coopw_solve(const GmCoopWArgs& a, int c, unsigne
       reason = -2;
       break;
     }
-    if (!xc_sync<X2>(a.sync, a.P, c, ++bk, s_err)) break;  // every workgroup's rows of x before the next residual
+    // every workgroup's rows of x before the next residual; then what is left
+    // of the last steps' exchange values is cleared (before the residual's
+    // barrier)
+    if (!xc_sync<X2>(a.sync, P, c, ++bk, s_err)) break;
+    for (int k = 0; k < 3; ++k) coopw_clear<X2>(a, c, r0, Rc, k, min(it, kmax + 1), gm_opaque(threadIdx.x), T);
   }
   if (threadIdx.x == 0) {
     if (*s_err) {
@@ -1779,70 +1530,63 @@ __device__ __forceinline__ void coopw_solve(const GmCoopWArgs& a, int c, unsigne
 
 // One cooperative solve by the workgroup of rank c (of a.P, all on one XCD
 // when the XCD ids they publish at the first barrier agree).
-template <int CQ>
+template <int RW, int CQ>
 __device__ __forceinline__ void coopw_run(const GmCoopWArgs& a, int c, double* dyn, double* red, double* s_val,
                                           int* s_flag, int* s_err) {
   if (threadIdx.x == 0) {
     *s_err = 0;
     __hip_atomic_store(a.sync + kXccSlot + c, gw_xcc_id() + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
+  for (int k = 0; k < 3; ++k)
+    coopw_clear<false>(a, c, c * a.R, min(a.nf, (c + 1) * a.R) - c * a.R, k, a.kmax + 1, threadIdx.x, kGmT);
   // barrier 1 at device scope; then every workgroup reads the P XCD ids
   // (the same values, so the same decision everywhere)
   if (xc_sync<false>(a.sync, a.P, c, 1u, s_err)) {
     if (threadIdx.x < 64) {
       const int lane = threadIdx.x;
-      const unsigned v =
-          lane < a.P ? __hip_atomic_load(a.sync + kXccSlot + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
+      const unsigned v = lane < a.P ? xc_ldu(a.sync + kXccSlot + lane) : 0u;
       const unsigned v0 = __builtin_amdgcn_readfirstlane(v);
       const bool same = a.l2x && __all(lane >= a.P || v == v0);
       if (lane == 0) s_flag[0] = same;
     }
     __syncthreads();
-    if (s_flag[0]) coopw_solve<CQ, true>(a, c, 1u, dyn, red, s_val, s_flag, s_err);
-    else coopw_solve<CQ, false>(a, c, 1u, dyn, red, s_val, s_flag, s_err);
+    if (s_flag[0]) coopw_solve<RW, CQ, true>(a, c, 1u, dyn, red, s_val, s_flag, s_err);
+    else coopw_solve<RW, CQ, false>(a, c, 1u, dyn, red, s_val, s_flag, s_err);
   } else if (threadIdx.x == 0) {
     a.s->reason = -3;
     a.s->its = 0;
   }
 }
 
-template <int CQ>
-__global__ void __launch_bounds__(kGmT) k_gmres_coopw(GmCoopWArgs a) {
-  __shared__ int s_c;
-  const int c = coop_rank(a.sync, a.P, a.xcd, &s_c);
-  if (c < 0) return;
-  extern __shared__ double dyn[];
-  __shared__ double red[2 * (kGmT / 64) + 1];
-  __shared__ double s_val[2];
-  __shared__ int s_flag[2];
-  __shared__ int s_err;
-  coopw_run<CQ>(a, c, dyn, red, s_val, s_flag, &s_err);
-}
-
-// Up to kCoopMulti solves in one launch, solve k on XCD a[k].xcd: the
-// workgroups on that XCD claim its ranks, those on XCDs no solve names, or
-// past a solve's P, leave at once.  Every XCD's workgroups belong to this
-// launch, so no solve waits for CUs another solve holds.
+// One solve, or up to kCoopMulti solves in one launch, solve k on XCD a[k].xcd
+// (P workgroups per XCD are launched): the workgroups on that XCD (XCC_ID)
+// claim its ranks in turn, those on XCDs no solve names, or past a solve's P,
+// leave at once.  Every XCD's workgroups belong to this launch, so no solve
+// waits for CUs another solve holds.  A single solve with xcd < 0 takes
+// workgroups 0, 8, 16, ... (one XCD when the dispatcher starts the launch's
+// round on it).
 constexpr int kCoopMulti = 8;
 struct GmCoopWMulti {
   int n;
   GmCoopWArgs a[kCoopMulti];
 };
 
-template <int CQ>
-__global__ void __launch_bounds__(kGmT) k_gmres_coopw_multi(GmCoopWMulti m) {
+template <int RW, int CQ>
+__global__ void __launch_bounds__(kGmT) k_gmres_coopw(GmCoopWMulti m) {
   __shared__ int s_c, s_k;
   if (threadIdx.x == 0) {
-    const int id = (int)gw_xcc_id();
-    int k = -1;
-    for (int j = 0; j < m.n; ++j)
-      if (m.a[j].xcd == id) k = j;
-    int c = -1;
-    if (k >= 0) {
-      c = (int)__hip_atomic_fetch_add(m.a[k].sync + kClaimSlot, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (c >= m.a[k].P) c = -1;
+    int k = -1, c = -1;
+    if (m.a[0].xcd < 0) {
+      k = 0;
+      if (blockIdx.x % 8 == 0) c = (int)(blockIdx.x / 8);
+    } else {
+      const int id = (int)gw_xcc_id();
+      for (int j = 0; j < m.n; ++j)
+        if (m.a[j].xcd == id) k = j;
+      if (k >= 0)
+        c = (int)__hip_atomic_fetch_add(m.a[k].sync + kClaimSlot, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    s_c = c;
+    s_c = k >= 0 && c < m.a[k].P ? c : -1;
     s_k = k;
   }
   __syncthreads();
@@ -1850,16 +1594,17 @@ __global__ void __launch_bounds__(kGmT) k_gmres_coopw_multi(GmCoopWMulti m) {
   if (c < 0) return;
   const int k = __builtin_amdgcn_readfirstlane(s_k);
   extern __shared__ double dyn[];
-  __shared__ double red[2 * (kGmT / 64) + 1];
+  __shared__ double red[kGmT / 64];
   __shared__ double s_val[2];
-  __shared__ int s_flag[2];
+  __shared__ int s_flag[3];
   __shared__ int s_err;
-  coopw_run<CQ>(m.a[k], c, dyn, red, s_val, s_flag, &s_err);
+  coopw_run<RW, CQ>(m.a[k], c, dyn, red, s_val, s_flag, &s_err);
 }
 
-// the barrier blocks of the launch's solves cleared and their statuses set
-// to reason -3 (one workgroup per solve)
-__global__ void k_coop_prep_multi(GmCoopWMulti m) {
+// before a cooperative launch: the barrier blocks of its solves cleared and
+// their statuses set to reason -3, which stays if no workgroup takes part (one
+// workgroup per solve)
+__global__ void k_coop_prep(GmCoopWMulti m) {
   const GmCoopWArgs& a = m.a[blockIdx.x];
   if (threadIdx.x < 2 * kCoopSyncDoubles) a.sync[threadIdx.x] = 0u;
   if (threadIdx.x == 0) {
@@ -1868,10 +1613,29 @@ __global__ void k_coop_prep_multi(GmCoopWMulti m) {
   }
 }
 
-// dynamic LDS of k_gmres_coopw without the basis (doubles): wl 32,
-// hcol/alpha kmax+2 each, lcc/lss kmax each, grs kmax+1, stg kCwBlk^2, ub nf
+// dynamic LDS of k_gmres_coopw without the basis (doubles): wl 64, nrm 32,
+// hcol/alpha kmax+2 each, grs kmax+1, stg kCwBlk kCwLd, ub nf
 static size_t coopw_lds_fixed(int nf, int kmax) {
-  return 32 + (size_t)5 * kmax + 5 + (size_t)kCwBlk * kCwBlk + (size_t)nf;
+  return 96 + (size_t)3 * kmax + 5 + (size_t)kCwBlk * kCwLd + (size_t)nf;
+}
+
+// The small form's split (nf <= 256, four rows per wavefront, the whole basis
+// in LDS): the fewest workgroups that hold it.
+constexpr int kCoopSmallQ = 4;
+
+bool gmres_coop_plan(int nf, int kmax, size_t max_lds, int* P, int* R) {
+  static const int cand[] = {2, 4, 8, 16, 32};
+  if (nf > 64 * kCoopSmallQ) return false;
+  for (int p : cand) {
+    const int r = (nf + p - 1) / p;
+    if (r < 1 || r > 4 * (kGmT / 64) || (p - 1) * r >= nf) continue;
+    if (kGmT / (kmax + 1) < 1) continue;
+    if (sizeof(double) * (coopw_lds_fixed(nf, kmax) + (size_t)(kmax + 1) * r) + 1024 > max_lds) continue;
+    *P = p;
+    *R = r;
+    return true;
+  }
+  return false;
 }
 
 bool gmres_coopw_plan(int nf, int kmax, size_t max_lds, int ncu, int* P, int* R, int* NL) {
@@ -1883,10 +1647,10 @@ bool gmres_coopw_plan(int nf, int kmax, size_t max_lds, int ncu, int* P, int* R,
   for (int p : cand) {
     if (8 * p > ncu) continue;
     const int r = (nf + p - 1) / p;
-    if (r > 2 * (kGmT / 64) || (p - 1) * r >= nf) continue;
+    if (r > 2 * (kGmT / 64)) continue;
     const long nl = std::min<long>(kmax + 1, (long)((budget - fixed) / r));
     if (nl < std::min(kmax + 1, 64)) continue;
-    *P = p;
+    *P = (nf + r - 1) / r;  // every workgroup has rows
     *R = r;
     *NL = (int)nl;
     return true;
@@ -1894,26 +1658,42 @@ bool gmres_coopw_plan(int nf, int kmax, size_t max_lds, int ncu, int* P, int* R,
   return false;
 }
 
+static int coopw_lpg(int P) {
+  int l = 0;
+  while ((1 << l) < P) ++l;
+  return l;
+}
+
+// Workspace (doubles), laid out by coopw_args.
 size_t gmres_coopw_ws(int nf, int kmax, int P, int R, int NL) {
-  return kCoopSyncDoubles + (size_t)P * (kmax + 2) + (size_t)4 * P + (size_t)nf + (size_t)(kmax + 1) * kmax +
-         (size_t)3 * (kmax + 1) + (size_t)P * R * (size_t)std::max(0, kmax + 1 - NL);
+  return kCoopSyncDoubles + ((size_t)3 * (kmax + 1) << coopw_lpg(P)) + (size_t)4 * (kmax + 1) + (size_t)4 * nf +
+         (size_t)2 * P + (size_t)(kmax + 1) * kmax + (size_t)3 * kmax + (size_t)P * R * (size_t)std::max(0, kmax + 1 - NL);
+}
+
+// The small form reserves what a Hessenberg copy per workgroup would take:
+// the size by which a caller's fixed workspace admits or refuses a solve.
+size_t gmres_coop_ws(int nf, int kmax, int P) {
+  const size_t reserved =
+      kCoopSyncDoubles + (size_t)P * (kmax + 2) + (size_t)4 * P + (size_t)nf + (size_t)P * (kmax + 1) * kmax;
+  return std::max(reserved, gmres_coopw_ws(nf, kmax, P, 0, kmax + 1));
 }
 
 // the kernel arguments of one solve, its workspace laid out in ws
 static GmCoopWArgs coopw_args(int nf, int kmax, int maxit, int P, int R, int NL, const double* S, const double* b,
                               double* x, GmresDev* s, double rtol, double atol, double* ws, int xcd) {
   GmCoopWArgs a{};
-  a.nf = nf; a.kmax = kmax; a.maxit = maxit; a.P = P; a.R = R; a.NL = NL; a.xcd = xcd;
+  a.nf = nf; a.kmax = kmax; a.maxit = maxit; a.P = P; a.lPg = coopw_lpg(P); a.R = R; a.NL = NL; a.xcd = xcd;
   a.S = S; a.b = b; a.x = x; a.s = s; a.rtol = rtol; a.atol = atol;
   a.sync = reinterpret_cast<unsigned*>(ws);
-  a.dots = ws + kCoopSyncDoubles;
-  a.norms = a.dots + (size_t)P * (kmax + 2);
-  a.wfull = a.norms + (size_t)4 * P;
-  a.Hg = a.wfull + nf;
-  a.yg = a.Hg + (size_t)(kmax + 1) * kmax;
-  a.hg = a.yg + (kmax + 1);
-  a.Rd = a.hg + (kmax + 1);
-  a.Vg = a.Rd + (kmax + 1);
+  a.x1 = ws + kCoopSyncDoubles;
+  a.x2 = a.x1 + ((size_t)3 * (kmax + 1) << a.lPg);
+  a.x3 = a.x2 + (size_t)3 * (kmax + 1);
+  a.rfull = a.x3 + (size_t)3 * nf;
+  a.norms = a.rfull + nf;
+  a.yg = a.norms + (size_t)2 * P;
+  a.Ht = a.yg + (kmax + 1);
+  a.rot = a.Ht + (size_t)(kmax + 1) * kmax;
+  a.Vg = a.rot + (size_t)3 * kmax;
   // IB_GMRES_L2_EXCHANGE=0 keeps the device-scope exchange even when every
   // workgroup is on one XCD (the results are the same bits either way)
   const char* e = std::getenv("IB_GMRES_L2_EXCHANGE");
@@ -1924,18 +1704,48 @@ static GmCoopWArgs coopw_args(int nf, int kmax, int maxit, int P, int R, int NL,
 // register columns per lane of the kernel instance for nf
 static int coopw_cq(int nf) { return nf <= 64 * 8 ? 8 : nf <= 64 * 13 ? 13 : 16; }
 
+static const void* coopw_kernel(int rw, int cq) {
+  if (rw == 4) return (const void*)k_gmres_coopw<4, kCoopSmallQ>;
+  return cq == 8 ? (const void*)k_gmres_coopw<2, 8>
+                 : cq == 13 ? (const void*)k_gmres_coopw<2, 13> : (const void*)k_gmres_coopw<2, 16>;
+}
+
+// the solves of m (one register layout) in one launch, P workgroups per XCD.
+// An ordinary launch: the barriers are the kernel's own (no runtime grid
+// synchronisation resources), one workgroup per CU; a workgroup that is not
+// resident in time makes the others leave with reason -3 instead of waiting
+// for ever.
+static void coopw_launch(hipStream_t st, int rw, const GmCoopWMulti& m, int nxcd) {
+  size_t lds = 0;
+  int maxP = 0;
+  for (int k = 0; k < m.n; ++k) {
+    const GmCoopWArgs& a = m.a[k];
+    lds = std::max(lds, sizeof(double) * (coopw_lds_fixed(a.nf, a.kmax) + (size_t)a.R * a.NL));
+    maxP = std::max(maxP, a.P);
+  }
+  // barrier words cleared by a kernel (a memset node misbehaves on graph replays)
+  hipLaunchKernelGGL(k_coop_prep, dim3(m.n), dim3(2 * kCoopSyncDoubles), 0, st, m);
+  IB_LAUNCH_CHECK();
+  const int nwg = (m.a[0].xcd < 0 ? 8 : std::max(nxcd, 1)) * maxP;
+  void* args[] = {(void*)&m};
+  IB_HIP(hipLaunchKernel(coopw_kernel(rw, coopw_cq(m.a[0].nf)), dim3(nwg), dim3(kGmT), args, lds, st));
+  IB_LAUNCH_CHECK();
+}
+
+void gmres_coop(hipStream_t st, int nf, int kmax, int maxit, int P, int R, const double* S, const double* b, double* x,
+                GmresDev* s, double rtol, double atol, double* ws, int xcd, int nxcd) {
+  GmCoopWMulti m{};
+  m.n = 1;
+  m.a[0] = coopw_args(nf, kmax, maxit, P, R, kmax + 1, S, b, x, s, rtol, atol, ws, xcd);
+  coopw_launch(st, 4, m, nxcd);
+}
+
 void gmres_coopw(hipStream_t st, int nf, int kmax, int maxit, int P, int R, int NL, const double* S, const double* b,
                  double* x, GmresDev* s, double rtol, double atol, double* ws, int xcd, int nxcd) {
-  const GmCoopWArgs a = coopw_args(nf, kmax, maxit, P, R, NL, S, b, x, s, rtol, atol, ws, xcd);
-  coop_prep(st, ws, s);
-  const size_t lds = sizeof(double) * (coopw_lds_fixed(nf, kmax) + (size_t)R * NL);
-  // P workgroups per XCD, of which the P on XCD xcd stay, one per CU
-  const int nwg = (xcd < 0 ? 8 : std::max(nxcd, 1)) * P;
-  const int cq = coopw_cq(nf);
-  if (cq == 8) hipLaunchKernelGGL(k_gmres_coopw<8>, dim3(nwg), dim3(kGmT), lds, st, a);
-  else if (cq == 13) hipLaunchKernelGGL(k_gmres_coopw<13>, dim3(nwg), dim3(kGmT), lds, st, a);
-  else hipLaunchKernelGGL(k_gmres_coopw<16>, dim3(nwg), dim3(kGmT), lds, st, a);
-  IB_LAUNCH_CHECK();
+  GmCoopWMulti m{};
+  m.n = 1;
+  m.a[0] = coopw_args(nf, kmax, maxit, P, R, NL, S, b, x, s, rtol, atol, ws, xcd);
+  coopw_launch(st, 2, m, nxcd);
 }
 
 bool gmres_coopw_multi_ok(int nf_a, int nf_b) { return coopw_cq(nf_a) == coopw_cq(nf_b); }
@@ -1945,23 +1755,12 @@ void gmres_coopw_multi(hipStream_t st, int n, const CoopWJob* jobs, const int* x
     throw HipError("gmres_coopw_multi: between 1 and min(8, XCDs) solves per launch");
   GmCoopWMulti m{};
   m.n = n;
-  size_t lds = 0;
-  int maxP = 0;
-  const int cq = coopw_cq(jobs[0].nf);
   for (int k = 0; k < n; ++k) {
     const CoopWJob& j = jobs[k];
-    if (coopw_cq(j.nf) != cq) throw HipError("gmres_coopw_multi: solves of different register layouts");
+    if (coopw_cq(j.nf) != coopw_cq(jobs[0].nf)) throw HipError("gmres_coopw_multi: solves of different register layouts");
     m.a[k] = coopw_args(j.nf, j.kmax, j.maxit, j.P, j.R, j.NL, j.S, j.b, j.x, j.s, j.rtol, j.atol, j.ws, xcds[k]);
-    lds = std::max(lds, sizeof(double) * (coopw_lds_fixed(j.nf, j.kmax) + (size_t)j.R * j.NL));
-    maxP = std::max(maxP, j.P);
   }
-  hipLaunchKernelGGL(k_coop_prep_multi, dim3(n), dim3(2 * kCoopSyncDoubles), 0, st, m);
-  IB_LAUNCH_CHECK();
-  const int nwg = std::max(nxcd, 1) * maxP;
-  if (cq == 8) hipLaunchKernelGGL(k_gmres_coopw_multi<8>, dim3(nwg), dim3(kGmT), lds, st, m);
-  else if (cq == 13) hipLaunchKernelGGL(k_gmres_coopw_multi<13>, dim3(nwg), dim3(kGmT), lds, st, m);
-  else hipLaunchKernelGGL(k_gmres_coopw_multi<16>, dim3(nwg), dim3(kGmT), lds, st, m);
-  IB_LAUNCH_CHECK();
+  coopw_launch(st, 2, m, nxcd);
 }
 
 // the kernel also has a few hundred bytes of static shared memory, so its
@@ -1970,20 +1769,12 @@ void gmres_dense_set_max_lds(size_t bytes) {
   if (bytes <= 1024) return;
   IB_HIP(hipFuncSetAttribute((const void*)k_gmres_dense<24>, hipFuncAttributeMaxDynamicSharedMemorySize,
                              (int)(bytes - 1024)));
-  IB_HIP(hipFuncSetAttribute((const void*)k_gmres_coop, hipFuncAttributeMaxDynamicSharedMemorySize,
-                             (int)(bytes - 1024)));
-  IB_HIP(hipFuncSetAttribute((const void*)k_gmres_coopw<8>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                             (int)(bytes - 1024)));
-  IB_HIP(hipFuncSetAttribute((const void*)k_gmres_coopw<13>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                             (int)(bytes - 1024)));
-  IB_HIP(hipFuncSetAttribute((const void*)k_gmres_coopw<16>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                             (int)(bytes - 1024)));
-  IB_HIP(hipFuncSetAttribute((const void*)k_gmres_coopw_multi<8>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                             (int)(bytes - 1024)));
-  IB_HIP(hipFuncSetAttribute((const void*)k_gmres_coopw_multi<13>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                             (int)(bytes - 1024)));
-  IB_HIP(hipFuncSetAttribute((const void*)k_gmres_coopw_multi<16>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                             (int)(bytes - 1024)));
+  const void* coop[] = {coopw_kernel(4, 0),
+                        coopw_kernel(2, 8),
+                        coopw_kernel(2, 13),
+                        coopw_kernel(2, 16)};
+  for (const void* f : coop)
+    IB_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(bytes - 1024)));
 }
 
 // ------------------------------------------------------------------------

@@ -801,7 +801,7 @@ struct ib_handle {
   // the status of a dense solve already copied to hst
   int dense_check() {
     if (cwP > 0 && coopP == 0) last_xmode = hst->xmode;
-    if (hst->reason == -3) return fail(IB_E_HIP, "GMRES: a grid barrier of the cooperative solve timed out");
+    if (hst->reason == -3) return fail(IB_E_HIP, "GMRES: a wait of the cooperative solve timed out");
     return hst->reason > 0 ? IB_OK : IB_E_NOCONV_GMRES;
   }
   int dense_status() {

@@ -459,19 +459,19 @@ void gmres_dense(hipStream_t st, int nf, int kmax, int maxit, const double* S, c
 void gmres_dense_set_max_lds(size_t bytes);
 bool gmres_dense_fits(int nf, int kmax, size_t max_lds);
 // The dense solve over P workgroups of one XCD (rows of S and of the basis
-// on chip, two grid barriers per step); plan: P and rows per workgroup R,
-// false if no split fits.  ws holds gmres_coop_ws doubles.  Status as
-// gmres_dense; reason -3: a grid barrier timed out.  xcd: the XCC id whose
+// on chip, the exchanged values polled by their readers); plan: P and rows per
+// workgroup R, false if no split fits.  ws holds gmres_coop_ws doubles.  Status
+// as gmres_dense; reason -3: a wait timed out.  xcd: the XCC id whose
 // workgroups run the solve (nxcd XCDs on the device), or -1 for workgroups
 // 0, 8, 16, ...
 bool gmres_coop_plan(int nf, int kmax, size_t max_lds, int* P, int* R);
 size_t gmres_coop_ws(int nf, int kmax, int P);
 void gmres_coop(hipStream_t st, int nf, int kmax, int maxit, int P, int R, const double* S, const double* b, double* x,
                 GmresDev* s, double rtol, double atol, double* ws, int xcd, int nxcd);
-// The dense solve over P workgroups of one XCD for nf <= 1024 and up to 1024
-// Krylov vectors (S rows in registers, basis rows in LDS up to NL vectors,
-// the rest in HBM; three grid barriers per step at most); plan: P, rows per
-// workgroup R and NL, false if no split fits.  ws holds gmres_coopw_ws doubles.
+// The same kernel's layout for nf <= 1024 and up to 1024 Krylov vectors (S
+// rows in registers, basis rows in LDS up to NL vectors, the rest in HBM);
+// plan: P, rows per workgroup R and NL, false if no split fits.  ws holds
+// gmres_coopw_ws doubles.
 // One solve of a fused launch of cooperative solves (gmres_coopw's
 // arguments); gmres_coopw_multi runs n <= min(8, nxcd) of them at once,
 // solve k on XCD xcds[k], provided gmres_coopw_multi_ok holds between their
