@@ -807,8 +807,11 @@ __device__ __forceinline__ void gc_wait_stores() { asm volatile("s_waitcnt vmcnt
 //    of vector j from conflict-free LDS reads, and the update w -= V h reads
 //    consecutive j across the lanes; vectors j >= NL (past the LDS) are kept
 //    in HBM in the same layout;
-//  * only workgroup 0 keeps the Hessenberg matrix (in HBM, unrotated, row by
-//    row) and runs the back substitution at the end of a cycle.
+//  * only workgroup 0 keeps the Hessenberg matrix (in HBM, row by row) and
+//    runs the back substitution at the end of a cycle.
+// Systems of up to 256 entries take four rows per wavefront and few workgroups
+// (the small form, RW = 4); it differs in the order of some sums and rotates
+// each new column at once by an affine scan.
 //
 // What bounds it is latency: an Arnoldi step is a chain of small products
 // joined by exchanges through L2.  So an exchanged value is its own flag: the
@@ -820,16 +823,18 @@ __device__ __forceinline__ void gc_wait_stores() { asm volatile("s_waitcnt vmcnt
 // sums coefficients c, c + P, ...; left out while every workgroup can load
 // all partials in two loads per thread) and the rows of the new vector u
 // (x3).  Everything that is not on that chain runs beside it:
-//  * u is exchanged and multiplied unnormalised (S v = S u / |u|), and every
-//    workgroup has the whole of it, so |u| is the last wavefront's, the same
-//    bits in every workgroup, while the others form S u;
+//  * every workgroup has the whole of the new vector u, exchanged
+//    unnormalised, so |u| is its own last wavefront's, the same bits
+//    everywhere, while the others form S u (S v = S u / |u|; the small form
+//    multiplies v itself, after |u|);
 //  * the Givens step and the stopping tests are the last wavefront's too,
 //    while the others form the dot products of S v.  A step's coefficients are
 //    therefore on their way before it is known whether the step before
 //    converged; after the last one they are not used;
 //  * entry it of the new column after the previous rotations is
 //    sum_j alpha_j h_j with alpha updated as [-s_it alpha, c_it], one dot
-//    product; the stored columns are rotated at the cycle's end.
+//    product; the stored columns are rotated at the cycle's end (small form:
+//    the scan, beside the update).
 // Each buffer has three copies, used in turn.  A workgroup clears what it
 // published in step s once it has published its rows of step s + 1 (its x2 of
 // that step was complete, which takes every workgroup's x1 of step s + 1, and
@@ -841,8 +846,9 @@ __device__ __forceinline__ void gc_wait_stores() { asm volatile("s_waitcnt vmcnt
 // Microseconds per Arnoldi step (events around the launches, start-up and
 // back substitution included), with grid barriers around each exchange and
 // now: airfoil + flap (nf = 800, ~460 steps a solve) 9.38 -> 6.55; plate (nf =
-// 202) 6.74 -> 4.83; flexible plate 6.69 -> 4.82; GMRES(30) of the cylinder
-// (nf = 314) 5.99 -> 3.56; a 42-entry system 5.77 -> 4.15.
+// 202) 6.74 -> 5.23; flexible plate 6.69 -> 5.26; GMRES(30) of the cylinder
+// (nf = 314) 5.99 -> 3.55; a 42-entry system 5.77 -> 4.28.  Both layouts round
+// as the kernels with grid barriers did (the solution's bits are theirs).
 // ------------------------------------------------------------------------
 constexpr int kCwBlk = 32;
 constexpr int kCwLd = kCwBlk + 1;  // row stride of a staged block (no bank conflicts down a column)
@@ -930,6 +936,13 @@ __device__ __forceinline__ double gw_block_sum(double v, double* red) {
   for (int q = 0; q < kGmT / 64; ++q) tot += red[q];
   __syncthreads();
   return tot;
+}
+
+// the sum over lanes 0..n-1 in that order (the whole wavefront must be active)
+__device__ __forceinline__ double gw_seq_sum(double v, int n) {
+  double t = 0.0;
+  for (int q = 0; q < n; ++q) t += gm_readlane(v, q);
+  return t;
 }
 
 // a product rounded by itself, whatever it is added to
@@ -1070,7 +1083,7 @@ __device__ __forceinline__ void coopw_clear(const GmCoopWArgs& a, int c, int r0,
 template <int RW, int CQ, bool X2>
 __device__ __forceinline__ void coopw_solve(const GmCoopWArgs& a, int c, unsigned bk, double* dyn, double* red,
                                             double* s_val, int* s_flag, int* s_err) {
-  constexpr int kLast = kGmT / 64 - 1;
+  constexpr bool kSmall = RW == 4;
   const int nf = a.nf, kmax = a.kmax, ld = kmax + 1, T = kGmT, R = a.R, NL = a.NL, P = a.P, lPg = a.lPg, Pg = 1 << lPg;
   const int r0 = c * R, Rc = min(nf, r0 + R) - r0;
   const int ldg = ld - NL;  // row stride of the basis vectors kept in HBM
@@ -1082,7 +1095,8 @@ __device__ __forceinline__ void coopw_solve(const GmCoopWArgs& a, int c, unsigne
   double* grs = alpha + kmax + 2;      // kmax + 1 (y of the back substitution in place)
   double* stg = grs + kmax + 1;        // kCwBlk x kCwLd: a diagonal block of the back substitution
   double* ub = stg + kCwBlk * kCwLd;   // nf: the vector of a product, u
-  double* Vl = ub + nf;                // R NL: local rows of basis vectors 0..NL-1, row-major
+  double* lss = ub + nf;               // small form, kmax: the rotations' sines (their cosines in alpha)
+  double* Vl = lss + (kSmall ? kmax : 0);  // R NL: local rows of basis vectors 0..NL-1, row-major
   // rows RW wq .. of S, columns ln + 64 k, in registers (0 outside the matrix)
   double s[RW][CQ];
   {
@@ -1097,13 +1111,13 @@ __device__ __forceinline__ void coopw_solve(const GmCoopWArgs& a, int c, unsigne
   }
   __syncthreads();
 
-  // wl = S[local rows] ub (wavefront q: rows RW q ..)
-  auto matvec = [&]() {
+  // wl = S[local rows] ub (small form: ub times scale) (wavefront q: rows RW q ..)
+  auto matvec = [&](double scale) {
     const int q = gm_opaque(threadIdx.x) >> 6, l = gm_opaque(threadIdx.x) & 63;
     if (RW * q < Rc) {  // uniform over the wavefront
       double v[CQ], acc[RW];
 #pragma unroll
-      for (int k = 0; k < CQ; ++k) v[k] = ub[min(l + 64 * k, nf - 1)];
+      for (int k = 0; k < CQ; ++k) v[k] = kSmall ? gw_mul(ub[min(l + 64 * k, nf - 1)], scale) : ub[min(l + 64 * k, nf - 1)];
 #pragma unroll
       for (int i = 0; i < RW; ++i) {
         acc[i] = 0.0;
@@ -1155,7 +1169,7 @@ __device__ __forceinline__ void coopw_solve(const GmCoopWArgs& a, int c, unsigne
     // ---- cycle start: r = b - S x (x from every workgroup's rows)
     for (int i = gm_opaque(threadIdx.x); i < nf; i += T) ub[i] = xc_ld(a.x + i);
     __syncthreads();
-    matvec();
+    matvec(1.0);
     __syncthreads();
     double pr = 0.0, pb = 0.0;
     for (int r = gm_opaque(threadIdx.x); r < Rc; r += T) {
@@ -1174,8 +1188,8 @@ __device__ __forceinline__ void coopw_solve(const GmCoopWArgs& a, int c, unsigne
     if (!xc_sync<X2>(a.sync, P, c, ++bk, s_err)) break;
     if (threadIdx.x < 64) {
       const int lane = threadIdx.x;
-      const double sr = gm_wave_sum(lane < P ? xc_ld(a.norms + lane * 2) : 0.0);
-      const double sb = gm_wave_sum(lane < P ? xc_ld(a.norms + lane * 2 + 1) : 0.0);
+      const double nr = lane < P ? xc_ld(a.norms + lane * 2) : 0.0, nb = lane < P ? xc_ld(a.norms + lane * 2 + 1) : 0.0;
+      const double sr = kSmall ? gw_seq_sum(nr, P) : gm_wave_sum(nr), sb = kSmall ? gw_seq_sum(nb, P) : gm_wave_sum(nb);
       if (lane == 0) {
         s_val[0] = sr;
         s_val[1] = sb;
@@ -1192,6 +1206,8 @@ __device__ __forceinline__ void coopw_solve(const GmCoopWArgs& a, int c, unsigne
     if (res0 == 0.0 || res0 <= ttol) reason = 1;
     else if (res0 >= 1e4 * rn0) reason = -1;
     if (reason) break;
+    if constexpr (kSmall)
+      for (int i = gm_opaque(threadIdx.x); i < nf; i += T) ub[i] = ub[i] / res0;
     __syncthreads();  // s_val is rewritten below
     int it = 0;         // columns formed
     int cur = 0, old = 2;  // it mod 3, (it - 1) mod 3
@@ -1201,11 +1217,28 @@ __device__ __forceinline__ void coopw_solve(const GmCoopWArgs& a, int c, unsigne
       // here ub = u, the unnormalised vector v_it
       const bool more = it < kmax && its < a.maxit;
       double tt = res0;  // last wavefront: |u|
-      matvec();
+      if constexpr (!kSmall) matvec(1.0);
       if (gm_opaque(threadIdx.x) >= T - 64) {
         const int lane = gm_opaque(threadIdx.x) & 63;
-        if (it > 0) tt = sqrt(gm_wave_sum(lane < P ? nrm[lane] : 0.0));
-        if (lane == 0) s_val[0] = 1.0 / tt;
+        if (it > 0) {
+          if constexpr (kSmall) {
+            // per workgroup its wavefronts' shares (stg) in turn, then the workgroups'
+            double v[16], t = 0.0;
+#pragma unroll
+            for (int q = 0; q < 16; ++q) v[q] = stg[16 * min(lane, P - 1) + q];
+#pragma unroll
+            for (int q = 0; q < 16; ++q) t += v[q];
+            tt = sqrt(gw_seq_sum(t, P));
+          } else {
+            tt = sqrt(gm_wave_sum(lane < P ? nrm[lane] : 0.0));
+          }
+        }
+        // the small form divides the residual itself (its u at it = 0 is v_0)
+        if (lane == 0) s_val[0] = kSmall && it == 0 ? 1.0 : 1.0 / tt;
+      }
+      if constexpr (kSmall) {
+        __syncthreads();
+        matvec(s_val[0]);
       }
       if (threadIdx.x == 0) s_flag[2] = *(volatile int*)s_err;
       __syncthreads();
@@ -1218,7 +1251,31 @@ __device__ __forceinline__ void coopw_solve(const GmCoopWArgs& a, int c, unsigne
       // rows: g lanes per j, lane sub takes rows sub, sub + g, ...; blocks of
       // four rows, the loads of a block ahead of its sums (the rows past Rc
       // add 0)
-      if (more) {
+      if constexpr (kSmall) {
+        // 16 lanes per coefficient, up to four rows each
+        if (more) {
+          const int t = gm_opaque(threadIdx.x), sub = t & 15;
+          double w[4];
+#pragma unroll
+          for (int q = 0; q < 4; ++q) w[q] = wl[min(sub + 16 * q, Rc - 1)];
+          for (int j0 = 0; j0 + ((t & ~63) >> 4) <= it; j0 += T / 16) {  // uniform over the wavefront
+            const int j = j0 + (t >> 4);
+            const double* vl = j < it ? Vl + j : ub + r0;  // v_it is not stored yet
+            const int ldv = j < it ? NL : 1;
+            const double sc = j < it ? 1.0 : inv;
+            double p = 0.0;
+            if (j <= it) {
+              double v[4];
+#pragma unroll
+              for (int q = 0; q < 4; ++q) v[q] = vl[min(sub + 16 * q, Rc - 1) * ldv];
+#pragma unroll
+              for (int q = 0; q < 4; ++q) p += (sub + 16 * q < Rc ? w[q] : 0.0) * gw_mul(v[q], sc);
+            }
+            p = gm_row_sum16(p);
+            if (j <= it && sub == 0) xc_put<X2>(a.x1 + ((cur * ld + j) << lPg) + c, p);
+          }
+        }
+      } else if (more) {
         const int lg = gw_log_lanes_per_coef(it), g = 1 << lg;
         const int t = gm_opaque(threadIdx.x), j = t >> lg, sub = t & (g - 1);
         if (((t & ~63) >> lg) <= it) {  // uniform over the wavefront
@@ -1276,7 +1333,7 @@ __device__ __forceinline__ void coopw_solve(const GmCoopWArgs& a, int c, unsigne
           const bool hap = tt < 1e-30 && tt < fabs(tt / gk);
           double res = 0.0, diag = hv;
           if (!hap) {
-            const double t1 = sqrt(hv * hv + tt * tt);
+            const double t1 = sqrt(kSmall ? __builtin_fma(tt, tt, gw_mul(hv, hv)) : __builtin_fma(hv, hv, gw_mul(tt, tt)));
             cc = hv / t1;
             sn = tt / t1;
             diag = cc * hv + sn * tt;
@@ -1290,7 +1347,11 @@ __device__ __forceinline__ void coopw_solve(const GmCoopWArgs& a, int c, unsigne
               grs[it] = -sn * gk;
               grs[k] = cc * gk;
             }
-            if (c == 0) {
+            if constexpr (kSmall) {
+              alpha[k] = cc;
+              lss[k] = sn;
+              if (c == 0) a.Ht[(long)k * kmax + k] = diag;
+            } else if (c == 0) {
               a.rot[3 * k] = cc;
               a.rot[3 * k + 1] = sn;
               a.rot[3 * k + 2] = diag;
@@ -1302,7 +1363,20 @@ __device__ __forceinline__ void coopw_solve(const GmCoopWArgs& a, int c, unsigne
       if (more) {
         const int n = it + 1;
         const double* x1 = a.x1 + ((cur * ld) << lPg);  // below 2^17
-        if ((n << lPg) <= 2 * T) {
+        if constexpr (kSmall) {
+          // every workgroup sums the partials of all (thread j coefficient j)
+          const int j = gm_opaque(threadIdx.x);
+          if ((j & ~63) < n) {  // uniform over the wavefront
+            const double* xj = x1 + (j << lPg);
+            double h = 0.0;
+            for (int q = 0; q < P; q += 2) {
+              const double2 v = xc_poll2(xj + q, j < n, xj + q + 1, j < n && q + 1 < P, a.sync, s_err);
+              h += v.x;
+              if (q + 1 < P) h += v.y;
+            }
+            if (j < n) hcol[j] = h;
+          }
+        } else if ((n << lPg) <= 2 * T) {
           // few partials: every workgroup sums all of them (Pg lanes per
           // coefficient, fixed butterfly)
           for (int base = 0; base < (n << lPg); base += T) {
@@ -1351,7 +1425,7 @@ __device__ __forceinline__ void coopw_solve(const GmCoopWArgs& a, int c, unsigne
           const int row = RW * q + gw_row<RW>(l);
           if (l < RW && row < Rc) {
             const double v = gw_mul(ub[r0 + row], inv);
-            xc_put<X2>(a.x3 + cur * nf + r0 + row, gw_mul(wl[row], inv) + sum);
+            xc_put<X2>(a.x3 + cur * nf + r0 + row, (kSmall ? wl[row] : gw_mul(wl[row], inv)) + sum);
             if (it < NL) Vl[row * NL + it] = v;
             else Vgc[(size_t)row * ldg + (it - NL)] = v;
           }
@@ -1362,6 +1436,23 @@ __device__ __forceinline__ void coopw_solve(const GmCoopWArgs& a, int c, unsigne
       }
       if (gm_opaque(threadIdx.x) >= T - 64) {
         const int lane = gm_opaque(threadIdx.x) & 63;
+        if constexpr (kSmall) {
+          // the previous rotations applied to the new column as an
+          // affine-recurrence scan, 64 rotations at a time
+          double carry = hcol[0];
+          for (int base = 0; base < it; base += 64) {
+            const int j = base + lane;
+            const bool act = j < it;
+            const double cj0 = act ? alpha[j] : 1.0, sj = act ? lss[j] : 0.0, hn = act ? hcol[j + 1] : 0.0;
+            double A = -sj, B = cj0 * hn;
+            gm_affine_scan(A, B);
+            const double cnext = A * carry + B;
+            const double cj = gm_shift_up1(cnext, carry);
+            if (act && c == 0) a.Ht[(long)j * kmax + it] = cj0 * cj + sj * hn;
+            carry = gm_readlane(cnext, min(63, it - 1 - base));
+          }
+          hv = carry;
+        } else {
         double part = 0.0;  // lane w: the sum over j = 64 w ..
 #pragma unroll 1
         for (int w0 = 0; 64 * w0 <= it; w0 += 4) {
@@ -1382,33 +1473,38 @@ __device__ __forceinline__ void coopw_solve(const GmCoopWArgs& a, int c, unsigne
           }
         }
         hv = gm_readlane(gm_row_sum16(part), 0);
+        }
       }
-      if (c == 0) {
+      if (!kSmall && c == 0) {
         for (int j = gm_opaque(threadIdx.x); j <= it; j += T) a.Ht[(long)j * kmax + it] = hcol[j];
       }
       ++it;
       ++its;
       old = cur;
       cur = cur == 2 ? 0 : cur + 1;
-      // the new vector, two adjacent rows of a workgroup per lane (16 lanes a
+      // the new vector, RW adjacent rows of a workgroup per lane (16 lanes a
       // workgroup), and the workgroups' shares of its squared norm: the
-      // squares of adjacent rows, then gm_row_sum16
+      // squares of the rows a wavefront owns, then gm_row_sum16 over the
+      // wavefronts (small form: one after the other, below)
       {
         const int t = gm_opaque(threadIdx.x), cq = t >> 4;
         if ((t >> 6) * 4 < P) {  // uniform over the wavefront
           const int rend = cq < P ? min(cq * R + R, nf) : 0;
-          double tot = 0.0;
-#pragma unroll
-          for (int b = 0; b < RW / 2; ++b) {
-            const int ra = cq * R + 32 * b + 2 * (t & 15);
-            const bool n0 = ra < rend, n1 = ra + 1 < rend;
-            const double* p = a.x3 + old * nf + ra;
-            const double2 u = xc_poll2(p, n0, p + 1, n1, a.sync, s_err);
-            if (n0) ub[ra] = u.x;
-            if (n1) ub[ra + 1] = u.y;
-            tot += gm_row_sum16(gw_mul(u.x, u.x) + gw_mul(u.y, u.y));
+          const int ra = cq * R + RW * (t & 15);
+          const double* p = a.x3 + old * nf + ra;
+          const double2 u = xc_poll2(p, ra < rend, p + 1, ra + 1 < rend, a.sync, s_err);
+          if (ra < rend) ub[ra] = u.x;
+          if (ra + 1 < rend) ub[ra + 1] = u.y;
+          if constexpr (kSmall) {
+            const double2 v = xc_poll2(p + 2, ra + 2 < rend, p + 3, ra + 3 < rend, a.sync, s_err);
+            if (ra + 2 < rend) ub[ra + 2] = v.x;
+            if (ra + 3 < rend) ub[ra + 3] = v.y;
+            if (cq < P)
+              stg[t] = (gw_mul(u.x, u.x) + gw_mul(v.x, v.x)) + (gw_mul(u.y, u.y) + gw_mul(v.y, v.y));
+          } else {
+            const double tot = gm_row_sum16(gw_mul(u.x, u.x) + gw_mul(u.y, u.y));
+            if ((t & 15) == 0 && cq < P) nrm[cq] = tot;
           }
-          if ((t & 15) == 0 && cq < P) nrm[cq] = tot;
         }
       }
       __syncthreads();
@@ -1418,6 +1514,7 @@ __device__ __forceinline__ void coopw_solve(const GmCoopWArgs& a, int c, unsigne
     // triangular system (grs becomes y in place) and publishes y
     const int top = it - 1;
     if (c == 0) {
+      if constexpr (!kSmall) {
       double* rc = hcol;   // the rotations (hcol and alpha are free here)
       double* rsn = alpha;
       for (int k = gm_opaque(threadIdx.x); k <= top; k += T) {
@@ -1446,6 +1543,7 @@ __device__ __forceinline__ void coopw_solve(const GmCoopWArgs& a, int c, unsigne
           }
         }
         col[(long)k * kmax] = a.rot[3 * k + 2];
+      }
       }
       __syncthreads();
       for (int kb1 = top; kb1 >= 0; kb1 -= kCwBlk) {
@@ -1490,7 +1588,24 @@ __device__ __forceinline__ void coopw_solve(const GmCoopWArgs& a, int c, unsigne
     for (int j = gm_opaque(threadIdx.x); j <= top; j += T) hcol[j] = xc_ld(a.yg + j);
     __syncthreads();
     // x += V y on the local rows
-    {
+    if constexpr (kSmall) {
+      const int r = gm_opaque(threadIdx.x);
+      if (r < Rc) {
+        double acc = 0.0;
+        for (int j0 = 0; j0 <= top; j0 += 8) {
+          double y[8], v[8];
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            y[i] = hcol[min(j0 + i, top)];
+            v[i] = Vl[r * NL + min(j0 + i, top)];
+          }
+#pragma unroll
+          for (int i = 0; i < 8; ++i)
+            if (j0 + i <= top) acc += y[i] * v[i];
+        }
+        xc_st<X2>(a.x + r0 + r, xc_ld(a.x + r0 + r) + acc);
+      }
+    } else {
       const int q = gm_opaque(threadIdx.x) >> 6, l = gm_opaque(threadIdx.x) & 63;
       if (RW * q < Rc) {
         double acc[RW];
@@ -1614,9 +1729,10 @@ __global__ void k_coop_prep(GmCoopWMulti m) {
 }
 
 // dynamic LDS of k_gmres_coopw without the basis (doubles): wl 64, nrm 32,
-// hcol/alpha kmax+2 each, grs kmax+1, stg kCwBlk kCwLd, ub nf
-static size_t coopw_lds_fixed(int nf, int kmax) {
-  return 96 + (size_t)3 * kmax + 5 + (size_t)kCwBlk * kCwLd + (size_t)nf;
+// hcol/alpha kmax+2 each, grs kmax+1, stg kCwBlk kCwLd, ub nf, and lss kmax in
+// the small form (rw = 4)
+static size_t coopw_lds_fixed(int rw, int nf, int kmax) {
+  return 96 + (size_t)(rw == 4 ? 4 : 3) * kmax + 5 + (size_t)kCwBlk * kCwLd + (size_t)nf;
 }
 
 // The small form's split (nf <= 256, four rows per wavefront, the whole basis
@@ -1630,7 +1746,7 @@ bool gmres_coop_plan(int nf, int kmax, size_t max_lds, int* P, int* R) {
     const int r = (nf + p - 1) / p;
     if (r < 1 || r > 4 * (kGmT / 64) || (p - 1) * r >= nf) continue;
     if (kGmT / (kmax + 1) < 1) continue;
-    if (sizeof(double) * (coopw_lds_fixed(nf, kmax) + (size_t)(kmax + 1) * r) + 1024 > max_lds) continue;
+    if (sizeof(double) * (coopw_lds_fixed(4, nf, kmax) + (size_t)(kmax + 1) * r) + 1024 > max_lds) continue;
     *P = p;
     *R = r;
     return true;
@@ -1642,7 +1758,7 @@ bool gmres_coopw_plan(int nf, int kmax, size_t max_lds, int ncu, int* P, int* R,
   static const int cand[] = {8, 16, 32};
   if (nf < 2 || nf > 64 * 16 || kmax < 1 || kmax + 1 > kGmT) return false;
   const size_t budget = max_lds > 2048 ? (max_lds - 2048) / sizeof(double) : 0;
-  const size_t fixed = coopw_lds_fixed(nf, kmax);
+  const size_t fixed = coopw_lds_fixed(2, nf, kmax);
   if (fixed >= budget) return false;
   for (int p : cand) {
     if (8 * p > ncu) continue;
@@ -1720,7 +1836,7 @@ static void coopw_launch(hipStream_t st, int rw, const GmCoopWMulti& m, int nxcd
   int maxP = 0;
   for (int k = 0; k < m.n; ++k) {
     const GmCoopWArgs& a = m.a[k];
-    lds = std::max(lds, sizeof(double) * (coopw_lds_fixed(a.nf, a.kmax) + (size_t)a.R * a.NL));
+    lds = std::max(lds, sizeof(double) * (coopw_lds_fixed(rw, a.nf, a.kmax) + (size_t)a.R * a.NL));
     maxP = std::max(maxP, a.P);
   }
   // barrier words cleared by a kernel (a memset node misbehaves on graph replays)
