@@ -299,6 +299,326 @@ __device__ __forceinline__ void load_twiddles(double2* Wl, const FFTPlan& pl) {
   for (int t = threadIdx.x; t < pl.L; t += blockDim.x) Wl[t] = pl.W[t];
 }
 
+// X_POINTROT: the patch of batch element by; false when this workgroup's rows
+// see no tap: they transform to zero, which is written
+__device__ __forceinline__ bool point_rows(const XArgs& a, PointPatch& pt, int by, int pair0, double* out) {
+  const int k = a.c0 + by;
+  // centre tap (p = l = 0) of force entry k, or face k of a face list
+  const int ck = a.w ? a.key[k * kTaps + kTaps / 2] : a.key[k];
+  const Geom& g = a.g;
+  const int N = a.pl.N, rp = a.rp, nrows = g.n - 1;
+  if (ck < g.Fx) { pt.comp = 1; pt.ix = ck % (g.m + 1) + 1; pt.iy = ck / (g.m + 1) + 1; }
+  else { pt.comp = 2; pt.ix = (ck - g.Fx) % g.m + 1; pt.iy = (ck - g.Fx) / g.m + 1; }
+  pt.w = a.w ? a.w + (long)k * kTaps : nullptr;
+  const int j0 = 2 * pair0 + 2, j1 = 2 * (pair0 + rp) + 1;  // node rows of this workgroup
+  if (j1 >= pt.iy - 3 && j0 <= pt.iy + 4) return true;
+  for (int idx = threadIdx.x; idx < rp * N; idx += blockDim.x) {
+    const int s = idx / N, t = idx - s * N;
+    const int ra = 2 * (pair0 + s), rb = ra + 1;
+    if (ra < nrows) out[(long)ra * N + t] = 0.0;
+    if (rb < nrows) out[(long)rb * N + t] = 0.0;
+  }
+  return false;
+}
+
+// The row pass's input at node (i, j).
+template <int MODE>
+__device__ __forceinline__ double row_value(const XArgs& a, const PointPatch& pt, const double* __restrict__ in,
+                                            const double* __restrict__ bc, int i, int j) {
+  const Geom& g = a.g;
+  double x;
+  if (MODE == X_POINTROT) {
+    x = pt.rot(i, j);
+  } else if (MODE == X_ROT) {
+    // rot_int + rot_bc: vort(i,j) = hy(i,j) - hy(i-1,j) - hx(i,j) + hx(i,j-1)
+    x = a.hy[(i - 1) + g.m * (j - 1)] - a.hy[(i - 2) + g.m * (j - 1)] - a.hx[(i - 1) + (g.m + 1) * (j - 1)] +
+        a.hx[(i - 1) + (g.m + 1) * (j - 2)];
+  } else {
+    x = in[(long)(j - 2) * (g.m - 1) + (i - 2)];
+  }
+  if (MODE == X_APPLYBC) {
+    // apply_bc(vort, sbc, 1.d0), src/operators_fluid.F90:539-549
+    if (i == 2) x = x + bc[g.left + j - 1];
+    if (i == g.m) x = x + bc[g.right + j - 1];
+    if (j == 2) x = x + bc[g.bottom + i - 1];
+    if (j == g.n) x = x + bc[g.top + i - 1];
+  }
+  return x;
+}
+
+// ------------------------------------------------------------------------
+// The passes with register ends, for plans of the fixed radices.  The
+// arithmetic is that of the passes below (the same radices, twiddles and order,
+// the same bits); what differs is what goes through LDS:
+//  * the first stage (radix 8: M is a multiple of 4) reads its eight inputs
+//    straight from the field, the second half as the odd extension's mirror
+//    (its twiddles are all 1), and the last stage stores the M - 1 values that
+//    are wanted straight to the field, so a transform of S stages makes S - 1
+//    trips through LDS instead of S + 1;
+//  * index i of a transform lies at i + i/8, which spreads the strided writes of
+//    a stage over the banks (the first radix-8 stage wrote eight lanes deep
+//    into one);
+//  * the twiddles come from the table in memory (L1), not from a copy in LDS,
+//    so a workgroup's LDS holds the two buffers only and a CU more workgroups;
+//  * an index is split by a multiplication (div_by), not a division.
+// What bounds them: a single field has at most 256 workgroups, one round of the
+// chip, and waits on a chain of a dozen barriers and loads; a batch has its
+// instructions, half of them addresses, at five wavefronts per SIMD (89
+// registers).  Us per field, plain form -> this one: one field, rows of 400
+// points 7.9 -> 6.4, of 1024 11.5 -> 8.1, columns of 400 13.3 -> 11.1, of 512
+// 18.7 -> 15.0; a batch of 8 -> of 32 fields, rows of 200 1.13 -> 0.40, of 400
+// 2.29 -> 1.09, columns of 200 1.95 -> 0.79, of 400 4.34 -> 2.67.
+// ------------------------------------------------------------------------
+__device__ __forceinline__ int pd(int i) { return i + (i >> 3); }
+__host__ __device__ inline int pd_len(int L) { return L + (L >> 3) + 1; }
+// i / d by the multiplier floor(2^32 / d) + 1: exact while i d < 2^32
+__device__ __forceinline__ int div_by(int i, unsigned mul) { return (int)__umulhi((unsigned)i, mul); }
+__device__ __forceinline__ double2 tw_at(const double2* __restrict__ W, int byte_off) {
+  return *(const double2*)((const char*)W + (unsigned)byte_off);
+}
+
+// butterfly j of a stage after the first, its inputs from a padded transform at
+// ip = transform + pd(j), twiddled.  LR and Ns are multiples of 8 there (the
+// first radix is 8), so pd(j + r LR) = pd(j) + r pd(LR).
+template <int R>
+__device__ __forceinline__ void bfly(const double2* __restrict__ ip, int pLR, int ktws,
+                                     const double2* __restrict__ W, double2* v) {
+  v[0] = ip[0];
+  const int kb = ktws * (int)sizeof(double2);
+#pragma unroll
+  for (int r = 1; r < R; ++r) v[r] = cmul(ip[r * pLR], tw_at(W, r * kb));
+  dft<R>(v);
+}
+
+template <int R>
+__device__ __forceinline__ void stage_pd(const double2* __restrict__ in, double2* __restrict__ out, int nf,
+                                         const FFTPlan& pl, int st, int Lp, int Ns) {
+  const int LR = pl.L / R, tws = LR / Ns, pLR = pd(LR), pNs = pd(Ns), total = nf * LR;
+  const unsigned mLR = pl.mLR[st], mNs = pl.mNs[st];
+  for (int idx = threadIdx.x; idx < total; idx += blockDim.x) {
+    const int s = div_by(idx, mLR), j = idx - s * LR, q = div_by(j, mNs), k = j - q * Ns;
+    double2 v[R];
+    bfly<R>(in + s * Lp + pd(j), pLR, k * tws, pl.W, v);
+    double2* op = out + s * Lp + pd(q * Ns * R + k);
+#pragma unroll
+    for (int r = 0; r < R; ++r) op[r * pNs] = v[r];
+  }
+}
+
+// stages 1 .. nst - 2 (the first is done, the last is the caller's), with a
+// barrier after each; returns the buffer that holds the result
+__device__ __forceinline__ double2* mid_stages(double2* a, double2* b, int nf, const FFTPlan& pl, int Lp) {
+  int Ns = 8;
+  for (int st = 1; st + 1 < pl.nst; ++st) {
+    const int R = pl.rad[st];
+    switch (R) {
+      case 8: stage_pd<8>(a, b, nf, pl, st, Lp, Ns); break;
+      case 4: stage_pd<4>(a, b, nf, pl, st, Lp, Ns); break;
+      case 2: stage_pd<2>(a, b, nf, pl, st, Lp, Ns); break;
+      case 3: stage_pd<3>(a, b, nf, pl, st, Lp, Ns); break;
+      default: stage_pd<5>(a, b, nf, pl, st, Lp, Ns); break;
+    }
+    __syncthreads();
+    double2* t = a;
+    a = b;
+    b = t;
+    Ns *= R;
+  }
+  return a;
+}
+
+// the eight inputs of first-stage butterfly j: z_t = x_t for t < M, 0 at t = 0
+// and M, -x_(2M-t) above; x(t) the field's value for t = 1 .. M - 1
+template <class X>
+__device__ __forceinline__ void load_first(double2* v, int j, int LR, int M, X&& x) {
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int t = j + r * LR;
+    const double2 p = x(t == 0 ? 1 : t), q = x(t == 0 ? 1 : M - t);
+    v[r] = t == 0 ? make_double2(0.0, 0.0) : p;
+    v[r + 4] = t == 0 ? make_double2(0.0, 0.0) : make_double2(-q.x, -q.y);
+  }
+}
+
+// the last stage: out(s, p, value) for p = 1 .. M - 1 of every transform; the
+// index runs over the transforms first where T is set (columns: adjacent
+// transforms are adjacent in memory)
+__device__ __forceinline__ int nf_shift(int nf) { return __ffs(nf) - 1; }
+template <int R, bool T, class OUT>
+__device__ __forceinline__ void last_stage_r(const double2* __restrict__ Z, int nf, const FFTPlan& pl, int Lp, OUT&& out) {
+  const int LR = pl.L / R, pLR = pd(LR);
+  const unsigned mLR = pl.mLR[pl.nst - 1];
+  for (int idx = threadIdx.x; idx < nf * LR; idx += blockDim.x) {
+    int s, k;
+    if (T) {
+      k = idx >> nf_shift(nf);
+      s = idx & (nf - 1);
+    } else {
+      s = div_by(idx, mLR);
+      k = idx - s * LR;
+    }
+    double2 v[R];
+    bfly<R>(Z + s * Lp + pd(k), pLR, k, pl.W, v);
+#pragma unroll
+    for (int r = 0; r < (R + 1) / 2; ++r) {
+      const int p = k + r * LR;
+      if (p >= 1 && p < pl.M) out(s, p, v[r]);
+    }
+  }
+}
+template <bool T, class OUT>
+__device__ __forceinline__ void last_stage(const double2* Z, int nf, const FFTPlan& pl, int Lp, OUT&& out) {
+  switch (pl.rad[pl.nst - 1]) {
+    case 8: last_stage_r<8, T>(Z, nf, pl, Lp, out); break;
+    case 4: last_stage_r<4, T>(Z, nf, pl, Lp, out); break;
+    case 2: last_stage_r<2, T>(Z, nf, pl, Lp, out); break;
+    case 3: last_stage_r<3, T>(Z, nf, pl, Lp, out); break;
+    default: last_stage_r<5, T>(Z, nf, pl, Lp, out); break;
+  }
+}
+
+template <int MODE>
+__device__ __forceinline__ void dst_xr_tile(const XArgs& a, int bx, int by) {
+  extern __shared__ double2 sm[];
+  const FFTPlan& pl = a.pl;
+  const int L = pl.L, N = pl.N, rp = a.rp, Lp = pd_len(L);
+  const int nrows = a.g.n - 1;
+  double2* A = sm;
+  double2* B = sm + rp * Lp;
+  const int bsel = a.strided ? 0 : by;
+  const double* __restrict__ in = a.in[bsel] ? a.in[bsel] + (long)by * a.s_in : nullptr;
+  double* out = a.out[bsel] + (long)by * a.s_out;
+  const double* bcb = a.bc ? a.bc + (long)by * a.s_bc : nullptr;
+  const int pair0 = bx * rp;
+  PointPatch pt{};
+  if (MODE == X_POINTROT && !point_rows(a, pt, by, pair0, out)) return;
+  const int LR = L / 8;
+  for (int idx = threadIdx.x; idx < rp * LR; idx += blockDim.x) {
+    const int s = div_by(idx, pl.mLR[0]), j = idx - s * LR;
+    const int ra = 2 * (pair0 + s), rb = ra + 1;
+    double2 v[8];
+    load_first(v, j, LR, pl.M, [&](int t) {
+      return make_double2(ra < nrows ? row_value<MODE>(a, pt, in, bcb, t + 1, ra + 2) : 0.0,
+                          rb < nrows ? row_value<MODE>(a, pt, in, bcb, t + 1, rb + 2) : 0.0);
+    });
+    dft<8>(v);
+#pragma unroll
+    for (int r = 0; r < 8; ++r) A[s * Lp + 9 * j + r] = v[r];
+  }
+  __syncthreads();
+  const double2* Z = mid_stages(A, B, rp, pl, Lp);
+  last_stage<false>(Z, rp, pl, Lp, [&](int s, int p, double2 z) {
+    const int ra = 2 * (pair0 + s), rb = ra + 1;
+    const long oa = (long)ra * N + p - 1, ob = (long)rb * N + p - 1;
+    if (MODE == X_SUBFROM) {
+      if (ra < nrows) out[oa] = out[oa] - (-z.y);
+      if (rb < nrows) out[ob] = out[ob] - z.x;
+    } else {
+      if (ra < nrows) out[oa] = -z.y;
+      if (rb < nrows) out[ob] = z.x;
+    }
+  });
+}
+
+template <int MODE>
+__device__ __forceinline__ void dst_yr_tile(const YArgs& a, int bx, int by) {
+  extern __shared__ double2 sm[];
+  const FFTPlan& pl = a.pl;
+  const int L = pl.L, M = pl.M, cp = a.cp, Lp = pd_len(L);
+  const int ncols = a.g.m - 1;
+  const int nfft = (MODE == Y_PRED) ? 2 * cp : cp;
+  double2* A = sm;
+  double2* B = sm + nfft * Lp;
+  const int bsel = a.strided ? 0 : by;
+  const double* __restrict__ in = a.in[bsel] + (long)by * a.s_in;
+  const double* __restrict__ in2 = a.in2[bsel] ? a.in2[bsel] + (long)by * a.s_in2 : nullptr;
+  double* __restrict__ out = a.out[bsel] + (long)by * a.s_out;
+  const int tile = (bx % 8) * a.chunk + bx / 8;  // a contiguous band of column tiles per XCD
+  const int col0 = 2 * tile * cp;
+  if (col0 >= ncols) return;
+  const int LR = L / 8;
+  for (int idx = threadIdx.x; idx < cp * LR; idx += blockDim.x) {
+    const int s = idx & (cp - 1), j = idx >> nf_shift(cp);
+    const int ca = col0 + 2 * s, cb = ca + 1;
+    double2 v[8];
+#pragma unroll
+    for (int q = 0; q < (MODE == Y_PRED ? 2 : 1); ++q) {
+      const double* __restrict__ f = q ? in2 : in;
+      load_first(v, j, LR, M, [&](int t) {
+        return make_double2(ca < ncols ? f[(long)(t - 1) * ncols + ca] : 0.0,
+                            cb < ncols ? f[(long)(t - 1) * ncols + cb] : 0.0);
+      });
+      dft<8>(v);
+#pragma unroll
+      for (int r = 0; r < 8; ++r) A[(s + q * cp) * Lp + 9 * j + r] = v[r];
+    }
+  }
+  __syncthreads();
+  double2* Z = mid_stages(A, B, nfft, pl, Lp);
+  if (MODE != Y_PLAIN) {
+    // the spectral product, extended oddly into the other buffer
+    double2* O = (Z == A) ? B : A;
+    const auto put = [&](int s, int p, double ya, double yb) {
+      O[s * Lp + pd(p)] = make_double2(ya, yb);
+      O[s * Lp + pd(L - p)] = make_double2(-ya, -yb);
+    };
+    if (MODE == Y_SCALE2) {
+      last_stage<true>(Z, cp, pl, Lp, [&](int s, int p, double2 z) {
+        const int ca = col0 + 2 * s, cb = ca + 1;
+        const double ya = (ca < ncols) ? a.tab[(long)(p - 1) * ncols + ca] * -z.y / a.div : 0.0;
+        const double yb = (cb < ncols) ? a.tab[(long)(p - 1) * ncols + cb] * z.x / a.div : 0.0;
+        put(s, p, ya, yb);
+      });
+    } else {
+      // the second field's spectrum first, into the other buffer's second half
+      double2* O2 = O + cp * Lp;
+      last_stage<true>(Z + cp * Lp, cp, pl, Lp, [&](int s, int p, double2 z) { O2[s * Lp + pd(p)] = z; });
+      __syncthreads();
+      last_stage<true>(Z, cp, pl, Lp, [&](int s, int p, double2 z) {
+        const int ca = col0 + 2 * s, cb = ca + 1;
+        const double2 zb = O2[s * Lp + pd(p)];
+        const double ba = -zb.y, bb = zb.x;
+        double ya = -z.y, yb = z.x;
+        // lam1i * (dst(rhs terms) + lam1 * dst(omega)), src/operators_fluid.F90:657-661
+        ya = (ca < ncols) ? a.tab2[(long)(p - 1) * ncols + ca] * (ya + a.tab[(long)(p - 1) * ncols + ca] * ba) : 0.0;
+        yb = (cb < ncols) ? a.tab2[(long)(p - 1) * ncols + cb] * (yb + a.tab[(long)(p - 1) * ncols + cb] * bb) : 0.0;
+        put(s, p, ya, yb);
+      });
+    }
+    for (int s = threadIdx.x; s < cp; s += blockDim.x) {
+      O[s * Lp] = make_double2(0.0, 0.0);
+      O[s * Lp + pd(M)] = make_double2(0.0, 0.0);
+    }
+    __syncthreads();
+    double2* Q = (O == A) ? B : A;
+    for (int idx = threadIdx.x; idx < cp * LR; idx += blockDim.x) {
+      const int s = div_by(idx, pl.mLR[0]), j = idx - s * LR;
+      double2 v[8];
+#pragma unroll
+      for (int r = 0; r < 8; ++r) v[r] = O[s * Lp + pd(j + r * LR)];
+      dft<8>(v);
+#pragma unroll
+      for (int r = 0; r < 8; ++r) Q[s * Lp + 9 * j + r] = v[r];
+    }
+    __syncthreads();
+    Z = mid_stages(Q, O, cp, pl, Lp);
+  }
+  last_stage<true>(Z, cp, pl, Lp, [&](int s, int p, double2 z) {
+    const int ca = col0 + 2 * s, cb = ca + 1;
+    if (ca < ncols) out[(long)(p - 1) * ncols + ca] = -z.y;
+    if (cb < ncols) out[(long)(p - 1) * ncols + cb] = z.x;
+  });
+}
+
+template <int MODE>
+__global__ void __launch_bounds__(512) k_dst_xr(XArgs a) {
+  dst_xr_tile<MODE>(a, blockIdx.x, blockIdx.y);
+}
+template <int MODE>
+__global__ void __launch_bounds__(512) k_dst_yr(YArgs a) {
+  dst_yr_tile<MODE>(a, blockIdx.x, blockIdx.y);
+}
+
 // Row pass.  Rows j0 = 0..n-2 (node j = j0+2) of length N = m-1.
 template <int MODE, bool GEN>
 __device__ __forceinline__ void dst_x_tile(const XArgs& a, int bx, int by) {
@@ -315,74 +635,14 @@ __device__ __forceinline__ void dst_x_tile(const XArgs& a, int bx, int by) {
   const double* bcb = a.bc ? a.bc + (long)by * a.s_bc : nullptr;
   const int pair0 = bx * rp;
   PointPatch pt{};
-  if (MODE == X_POINTROT) {
-    const int k = a.c0 + by;
-    // centre tap (p = l = 0) of force entry k, or face k of a face list
-    const int ck = a.w ? a.key[k * kTaps + kTaps / 2] : a.key[k];
-    const Geom& g = a.g;
-    if (ck < g.Fx) { pt.comp = 1; pt.ix = ck % (g.m + 1) + 1; pt.iy = ck / (g.m + 1) + 1; }
-    else { pt.comp = 2; pt.ix = (ck - g.Fx) % g.m + 1; pt.iy = (ck - g.Fx) / g.m + 1; }
-    pt.w = a.w ? a.w + (long)k * kTaps : nullptr;
-    // rows whose nodes see no tap transform to zero: write zeros and leave
-    const int j0 = 2 * pair0 + 2, j1 = 2 * (pair0 + rp) + 1;  // node rows of this workgroup
-    if (j1 < pt.iy - 3 || j0 > pt.iy + 4) {
-      for (int idx = threadIdx.x; idx < rp * N; idx += blockDim.x) {
-        const int s = idx / N, t = idx - s * N;
-        const int ra = 2 * (pair0 + s), rb = ra + 1;
-        if (ra < nrows) out[(long)ra * N + t] = 0.0;
-        if (rb < nrows) out[(long)rb * N + t] = 0.0;
-      }
-      return;
-    }
-  }
+  if (MODE == X_POINTROT && !point_rows(a, pt, by, pair0, out)) return;
   load_twiddles(Wl, pl);
   for (int idx = threadIdx.x; idx < rp * N; idx += blockDim.x) {
     const int s = idx / N;
     const int t = idx - s * N;
     const int ra = 2 * (pair0 + s), rb = ra + 1;
-    double xa = 0.0, xb = 0.0;
-    if (MODE == X_POINTROT) {
-      const int i = t + 2;
-      if (ra < nrows) xa = pt.rot(i, ra + 2);
-      if (rb < nrows) xb = pt.rot(i, rb + 2);
-    } else if (MODE == X_ROT) {
-      // rot_int + rot_bc: vort(i,j) = hy(i,j) - hy(i-1,j) - hx(i,j) + hx(i,j-1)
-      const Geom& g = a.g;
-      const int i = t + 2;
-      if (ra < nrows) {
-        const int j = ra + 2;
-        xa = a.hy[(i - 1) + g.m * (j - 1)] - a.hy[(i - 2) + g.m * (j - 1)] - a.hx[(i - 1) + (g.m + 1) * (j - 1)] +
-             a.hx[(i - 1) + (g.m + 1) * (j - 2)];
-      }
-      if (rb < nrows) {
-        const int j = rb + 2;
-        xb = a.hy[(i - 1) + g.m * (j - 1)] - a.hy[(i - 2) + g.m * (j - 1)] - a.hx[(i - 1) + (g.m + 1) * (j - 1)] +
-             a.hx[(i - 1) + (g.m + 1) * (j - 2)];
-      }
-    } else {
-      if (ra < nrows) xa = in[(long)ra * N + t];
-      if (rb < nrows) xb = in[(long)rb * N + t];
-    }
-    if (MODE == X_APPLYBC) {
-      // apply_bc(vort, sbc, 1.d0), src/operators_fluid.F90:539-549
-      const int i = t + 2;
-      const Geom& g = a.g;
-      const double* bc = bcb;
-      if (ra < nrows) {
-        const int j = ra + 2;
-        if (i == 2) xa = xa + bc[g.left + j - 1];
-        if (i == g.m) xa = xa + bc[g.right + j - 1];
-        if (j == 2) xa = xa + bc[g.bottom + i - 1];
-        if (j == g.n) xa = xa + bc[g.top + i - 1];
-      }
-      if (rb < nrows) {
-        const int j = rb + 2;
-        if (i == 2) xb = xb + bc[g.left + j - 1];
-        if (i == g.m) xb = xb + bc[g.right + j - 1];
-        if (j == 2) xb = xb + bc[g.bottom + i - 1];
-        if (j == g.n) xb = xb + bc[g.top + i - 1];
-      }
-    }
+    const double xa = ra < nrows ? row_value<MODE>(a, pt, in, bcb, t + 2, ra + 2) : 0.0;
+    const double xb = rb < nrows ? row_value<MODE>(a, pt, in, bcb, t + 2, rb + 2) : 0.0;
     A[s * L + t + 1] = make_double2(xa, xb);
     A[s * L + L - (t + 1)] = make_double2(-xa, -xb);
   }
@@ -544,7 +804,12 @@ void HostFFTPlan::init(int N) {
   std::vector<int> rad = factorize(dev.L);
   if ((int)rad.size() > kMaxStages) throw HipError("FFT length has too many factors");
   dev.nst = (int)rad.size();
-  for (int i = 0; i < dev.nst; ++i) dev.rad[i] = rad[i];
+  for (int i = 0, ns = 1; i < dev.nst; ns *= rad[i++]) {
+    dev.rad[i] = rad[i];
+    if (i >= kRegStages) continue;
+    dev.mLR[i] = (unsigned)(0x100000000ull / (dev.L / rad[i])) + 1;
+    dev.mNs[i] = (unsigned)(0x100000000ull / ns) + 1;
+  }
   std::vector<double2> w(dev.L);
   for (int t = 0; t < dev.L; ++t) {
     long double ang = 2.0L * 3.14159265358979323846264338327950288L * (long double)t / (long double)dev.L;
@@ -561,6 +826,32 @@ void HostFFTPlan::release() {
 }
 
 size_t dst_lds_bytes(const FFTPlan& pl, int nfft) { return (size_t)(2 * nfft + 1) * pl.L * sizeof(double2); }
+
+static size_t reg_lds_bytes(const FFTPlan& pl, int nfft) { return (size_t)2 * nfft * pd_len(pl.L) * sizeof(double2); }
+// Whether a plan takes the passes with register ends: the fixed radices, and
+// above the lengths where a single field goes to the matrix cores instead.
+// There the plain form is what the matrix-core form is timed against, and a
+// faster one would turn near ties (us, one field, 200 points: rows 6.7 plain,
+// 5.4 matrix cores; 320: 7.7 and 7.6; columns, 200: 10.7 and 10.9); a strided
+// batch is 1.3 times faster without the matrix cores already at 200.
+static bool fft_reg_plan(const FFTPlan& pl, int from) {
+  return !fft_has_generic(pl) && pl.nst >= 2 && pl.nst <= kRegStages && pl.rad[0] == 8 && pl.M >= from;
+}
+constexpr int kRegRow = 320, kRegCol = 200, kRegBatch = 200;
+// a launch of tiles of `tile` pairs, nfft transforms in all (column passes
+// split an index by the tile with a shift)
+static bool fft_reg_ends(const FFTPlan& pl, int from, int tile, int nfft, size_t max_lds) {
+  return fft_reg_plan(pl, from) && (tile & (tile - 1)) == 0 && reg_lds_bytes(pl, nfft) <= max_lds;
+}
+// Threads: about four points each, so that a stage is one or two rounds.  Us per
+// field of a batch of 32, 128 / 256 / 512 threads: columns of 400 points, one
+// pair 2.96 / 2.67 / 4.06; of 512 points, two pairs 10.0 / 7.9 / 7.4; rows of
+// 400 points 1.19 / 1.09 / 1.60; one field's rows of 1024 points 10.4 / 8.6 / 8.1.
+static int reg_threads(const FFTPlan& pl, int nfft) { return nfft * pl.L >= 2048 ? 512 : 256; }
+// Pairs per workgroup of a strided batch: the most that keep it to 1280 points
+// (us per field of 32, rows + columns, 1 / 2 / 4 pairs: 200 points 1.30 / 1.19 /
+// 1.38, 320 x 240 2.25 / 1.78 / 2.19, 400 points 3.76 / 4.32 / 5.53).
+static int reg_batch_tile(const FFTPlan& pl) { return pl.L <= 320 ? 4 : (pl.L <= 640 ? 2 : 1); }
 
 bool fft_has_generic(const FFTPlan& pl) {
   for (int st = 0; st < pl.nst; ++st) {
@@ -582,6 +873,24 @@ const void* dst_x_kernel_t(int mode) {
     case X_ROT: return (const void*)k_dst_x<X_ROT, GEN>;
     case X_POINTROT: return (const void*)k_dst_x<X_POINTROT, GEN>;
     default: throw HipError("bad DST row mode");
+  }
+}
+const void* dst_xr_kernel(int mode) {
+  switch (mode) {
+    case X_PLAIN: return (const void*)k_dst_xr<X_PLAIN>;
+    case X_APPLYBC: return (const void*)k_dst_xr<X_APPLYBC>;
+    case X_SUBFROM: return (const void*)k_dst_xr<X_SUBFROM>;
+    case X_ROT: return (const void*)k_dst_xr<X_ROT>;
+    case X_POINTROT: return (const void*)k_dst_xr<X_POINTROT>;
+    default: throw HipError("bad DST row mode");
+  }
+}
+const void* dst_yr_kernel(int mode) {
+  switch (mode) {
+    case Y_PLAIN: return (const void*)k_dst_yr<Y_PLAIN>;
+    case Y_SCALE2: return (const void*)k_dst_yr<Y_SCALE2>;
+    case Y_PRED: return (const void*)k_dst_yr<Y_PRED>;
+    default: throw HipError("bad DST column mode");
   }
 }
 const void* dst_y_kernel(int mode) {
@@ -623,7 +932,11 @@ void dst_set_max_lds(size_t bytes) {
     for (int mode : {X_PLAIN, X_APPLYBC, X_SUBFROM, X_ROT, X_POINTROT}) fns.push_back(dst_x_kernel(mode, gen));
     for (int mode : {X_PLAIN, X_APPLYBC, X_SUBFROM, X_ROT}) fns.push_back(dst_x_tab_kernel(mode, gen));
   }
-  for (int mode : {Y_PLAIN, Y_SCALE2, Y_PRED}) fns.push_back(dst_y_kernel(mode));
+  for (int mode : {X_PLAIN, X_APPLYBC, X_SUBFROM, X_ROT, X_POINTROT}) fns.push_back(dst_xr_kernel(mode));
+  for (int mode : {Y_PLAIN, Y_SCALE2, Y_PRED}) {
+    fns.push_back(dst_y_kernel(mode));
+    fns.push_back(dst_yr_kernel(mode));
+  }
   for (int mode : {Y_SCALE2, Y_PRED}) fns.push_back(dst_y_tab_kernel(mode));
   for (const void* f : fns) IB_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
 }
@@ -700,7 +1013,11 @@ void dst_x(hipStream_t st, const FFTPlan& pl, int mode, const DstLaunch& l, cons
   size_t lds = 0;
   const TabEntry<XArgs> e = dst_x_entry(pl, l, g, rp, max_lds, &lds);
   void* args[] = {(void*)&e.a};
-  IB_HIP(hipLaunchKernel(dst_x_kernel(mode, fft_has_generic(pl)), dim3(e.nbx, e.nby), dim3(256), args, lds, st));
+  if (fft_reg_ends(pl, l.strided ? kRegBatch : kRegRow, e.a.rp, e.a.rp, max_lds))
+    IB_HIP(hipLaunchKernel(dst_xr_kernel(mode), dim3(e.nbx, e.nby), dim3(reg_threads(pl, e.a.rp)), args,
+                           reg_lds_bytes(pl, e.a.rp), st));
+  else
+    IB_HIP(hipLaunchKernel(dst_x_kernel(mode, fft_has_generic(pl)), dim3(e.nbx, e.nby), dim3(256), args, lds, st));
   IB_LAUNCH_CHECK();
 }
 
@@ -709,7 +1026,12 @@ void dst_y(hipStream_t st, const FFTPlan& pl, int mode, const DstLaunch& l, cons
   size_t lds = 0;
   const TabEntry<YArgs> e = dst_y_entry(pl, mode, l, g, cp, max_lds, &lds);
   void* args[] = {(void*)&e.a};
-  IB_HIP(hipLaunchKernel(dst_y_kernel(mode), dim3(e.nbx, e.nby), dim3(256), args, lds, st));
+  const int nfft = (mode == Y_PRED ? 2 : 1) * e.a.cp;
+  if (fft_reg_ends(pl, l.strided ? kRegBatch : kRegCol, e.a.cp, nfft, max_lds))
+    IB_HIP(hipLaunchKernel(dst_yr_kernel(mode), dim3(e.nbx, e.nby), dim3(reg_threads(pl, nfft)), args,
+                           reg_lds_bytes(pl, nfft), st));
+  else
+    IB_HIP(hipLaunchKernel(dst_y_kernel(mode), dim3(e.nbx, e.nby), dim3(256), args, lds, st));
   IB_LAUNCH_CHECK();
 }
 
@@ -724,7 +1046,9 @@ void dst_y(hipStream_t st, const FFTPlan& pl, int mode, const DstLaunch& l, cons
 // scratch fields between HIP events; the fastest is kept for the process,
 // per grid shape.  Two classes are timed: one field per launch (the time
 // step) and a strided batch of 8 fields (the Schur assembly, whose launches
-// cover hundreds of columns).
+// cover hundreds of columns).  The Stockham tiles are timed for one field; the
+// batch takes the same ones, or reg_batch_tile's for the passes with register
+// ends.
 //
 // IB_DST_TILES=rp,cp forces the Stockham tiles; IB_DST_TUNE=0 keeps the
 // fixed rule (rp 2 up to transform length 512, else 1; cp 1); neither times
@@ -795,6 +1119,7 @@ DstTiles dst_tiles(hipStream_t st, const FFTPlan& px, const FFTPlan& py, const D
   DstTiles t;
   t.rp = px.L <= 512 ? 2 : 1;
   t.cp = 1;
+  t.rp_b = t.rp;
   int forced_cfg = kDenseDefault;
   const int rule = form_rule(&forced_cfg);
   const bool dense_ok = dx && dy && dx->S && dy->S && tq;
@@ -806,6 +1131,8 @@ DstTiles dst_tiles(hipStream_t st, const FFTPlan& px, const FFTPlan& py, const D
       throw HipError("IB_DST_TILES must be rp,cp with 1 <= rp, cp <= 8");
     t.rp = rp;  // dst_x_entry / dst_y_entry halve a choice the LDS cannot hold
     t.cp = cp;
+    t.rp_b = rp;
+    t.cp_b = cp;
     t.xform = t.yform = t.xform_b = t.yform_b = fixed_form;
     t.source = 2;
     return t;
@@ -866,8 +1193,10 @@ DstTiles dst_tiles(hipStream_t st, const FFTPlan& px, const FFTPlan& py, const D
   DstLaunch by = bx;
   by.tab = in.p;
   by.div = 1.0;
-  t.us[4] = time_launches(st, [&] { dst_x(st, px, X_PLAIN, bx, g, t.rp, max_lds); }) * 1e3f / kTuneBatch;
-  t.us[6] = time_launches(st, [&] { dst_y(st, py, Y_SCALE2, by, g, t.cp, max_lds); }) * 1e3f / kTuneBatch;
+  t.rp_b = fft_reg_plan(px, kRegBatch) ? reg_batch_tile(px) : t.rp;
+  t.cp_b = fft_reg_plan(py, kRegBatch) ? reg_batch_tile(py) : t.cp;
+  t.us[4] = time_launches(st, [&] { dst_x(st, px, X_PLAIN, bx, g, t.rp_b, max_lds); }) * 1e3f / kTuneBatch;
+  t.us[6] = time_launches(st, [&] { dst_y(st, py, Y_SCALE2, by, g, t.cp_b, max_lds); }) * 1e3f / kTuneBatch;
   if (try_dense) {
     // a class is timed only if the matrix-core form could beat the measured
     // Stockham time at the FP64 matrix peak (78.6 TFLOP/s; 2N flops per

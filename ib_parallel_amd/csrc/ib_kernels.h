@@ -115,6 +115,7 @@ void dst_dense_y(hipStream_t st, const DenseMat& S, int mode, const DstLaunch& a
 // source: 0 fixed rule, 1 timed, 2 forced by IB_DST_TILES or IB_DST_FORM.
 struct DstTiles {
   int rp = 1, cp = 1, source = 0;
+  int rp_b = 1, cp_b = 1;  // of the batched class
   int xform = 0, yform = 0, xform_b = 0, yform_b = 0;
   float us[8] = {-1, -1, -1, -1, -1, -1, -1, -1};
 };
