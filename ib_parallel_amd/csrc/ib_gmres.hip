@@ -702,18 +702,20 @@ void gmres_dense(hipStream_t st, int nf, int kmax, int maxit, const double* S, c
 // below).  The launch has P workgroups per XCD, dealt by the dispatcher to
 // the XCDs in turn; the P on the XCD the host names take part, so
 // a solve keeps to one XCD's CUs and L2 and solves on different XCDs run side
-// by side.  All waits are bounded: on a timeout every workgroup leaves with
-// reason -3.
+// by side.  All waits are bounded: on a timeout the workgroups leave and the
+// status stays at reason -3.
 // ------------------------------------------------------------------------
 constexpr long kCoopSpin = 1L << 22;
 
 // The barrier block of a cooperative solve (unsigned words, cleared before
 // each launch): word 0 the error flag, 8.. the workgroups' barrier counts,
-// kXccSlot.. the XCD ids they publish, kClaimSlot the ranks claimed.
+// kXccSlot.. the XCD ids they publish, kClaimSlot the ranks claimed, kDoneSlot
+// the workgroups that have ended their part.
 constexpr int kCoopSyncDoubles = 40;
 constexpr int kXccSlot = 40;
 constexpr int kClaimSlot = 72;
-static_assert(kClaimSlot < 2 * kCoopSyncDoubles, "barrier block too small");
+constexpr int kDoneSlot = 73;
+static_assert(kDoneSlot < 2 * kCoopSyncDoubles, "barrier block too small");
 
 // The XCD this wavefront runs on (HW_REG_XCC_ID, bits 3:0).
 __device__ __forceinline__ unsigned gw_xcc_id() { return __builtin_amdgcn_s_getreg((3 << 11) | (0 << 6) | 20) & 0xFu; }
@@ -858,6 +860,7 @@ struct GmCoopWArgs {
   int nf, kmax, maxit, P, lPg, R, NL;  // Pg = 2^lPg: the power of two >= P
   int xcd;  // the XCD whose workgroups take part (-1: workgroups 0, 8, 16, ...)
   int l2x;  // 1: exchange through one XCD's L2 when every workgroup is found there
+  int fail_rank;  // the workgroup that takes its last wait of a cycle as timed out (-1: none)
   const double* S;
   const double* b;
   double* x;
@@ -1510,6 +1513,10 @@ __device__ __forceinline__ void coopw_solve(const GmCoopWArgs& a, int c, unsigne
       __syncthreads();
     }
     if (!ok) break;
+    if (c == a.fail_rank && threadIdx.x == 0) {  // as xc_give_up in the last step
+      __hip_atomic_store(a.sync, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      *s_err = 1;
+    }
     // ---- KSPGMRESBuildSoln: workgroup 0 rotates the columns, solves the
     // triangular system (grs becomes y in place) and publishes y
     const int top = it - 1;
@@ -1628,11 +1635,16 @@ __device__ __forceinline__ void coopw_solve(const GmCoopWArgs& a, int c, unsigne
     if (!xc_sync<X2>(a.sync, P, c, ++bk, s_err)) break;
     for (int k = 0; k < 3; ++k) coopw_clear<X2>(a, c, r0, Rc, k, min(it, kmax + 1), gm_opaque(threadIdx.x), T);
   }
+  // The last workgroup to end its part without a time-out reports the result
+  // (all hold the same one).  A workgroup that gives up raises its flag of the
+  // last barrier before the error word is looked at, and others may then pass
+  // that barrier; it is not counted, so the status stays the time-out that
+  // k_coop_prep wrote.
   if (threadIdx.x == 0) {
     if (*s_err) {
-      a.s->reason = -3;
       a.s->its = its;
-    } else if (c == 0) {
+    } else if (__hip_atomic_fetch_add(a.sync + kDoneSlot, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u ==
+               (unsigned)P) {
       a.s->its = its;
       a.s->reason = reason;
       a.s->rn0 = rn0;
@@ -1667,9 +1679,6 @@ __device__ __forceinline__ void coopw_run(const GmCoopWArgs& a, int c, double* d
     __syncthreads();
     if (s_flag[0]) coopw_solve<RW, CQ, true>(a, c, 1u, dyn, red, s_val, s_flag, s_err);
     else coopw_solve<RW, CQ, false>(a, c, 1u, dyn, red, s_val, s_flag, s_err);
-  } else if (threadIdx.x == 0) {
-    a.s->reason = -3;
-    a.s->its = 0;
   }
 }
 
@@ -1814,6 +1823,10 @@ static GmCoopWArgs coopw_args(int nf, int kmax, int maxit, int P, int R, int NL,
   // workgroup is on one XCD (the results are the same bits either way)
   const char* e = std::getenv("IB_GMRES_L2_EXCHANGE");
   a.l2x = e && std::atoi(e) == 0 ? 0 : 1;
+  // IB_GMRES_FAIL_RANK=c lets workgroup c time out at the end of a cycle (the
+  // tests' way to that path)
+  const char* f = std::getenv("IB_GMRES_FAIL_RANK");
+  a.fail_rank = f ? std::atoi(f) : -1;
   return a;
 }
 

@@ -7,7 +7,8 @@ import numpy as np
 import pytest
 
 from conftest import rel
-from ib_parallel_amd import decks
+from ib_parallel_amd import abi, decks
+from ib_parallel_amd.sim import IBError
 
 pytestmark = pytest.mark.gpu
 
@@ -81,3 +82,26 @@ def test_cooperative_gmres_from_the_solution():
     mk = lambda f: _circle(130, gmres_restart=30, gmres_form=f)
     x, its, r, info, _ = _solve(mk, 0, x0=1.0)
     assert info[0] == 3 and its == 0 and r < 1e-11
+
+
+@pytest.mark.parametrize("npts, form, groups", [(21, 2, 2), (130, 0, 16)])
+@pytest.mark.parametrize("exchange", ("1", "0"))
+def test_a_workgroup_that_gives_up_fails_the_solve(monkeypatch, npts, form, groups, exchange):
+    """A workgroup whose last wait times out leaves without its rows of the
+    solution: the solve reports the time-out, whichever workgroup it is and
+    although all the others finish, and the next solve on the handle is whole."""
+    from ib_parallel_amd import GpuSim
+    monkeypatch.setenv("IB_GMRES_L2_EXCHANGE", exchange)
+    g = GpuSim(*_circle(npts, gmres_restart=400, gmres_form=form))
+    assert g.gmres_info()[1] == groups
+    b = g.schur_matrix() @ np.random.default_rng(5).standard_normal(g.nf)
+    want = g.gmres(b)
+    for rank in (0, 1, groups - 1):
+        monkeypatch.setenv("IB_GMRES_FAIL_RANK", str(rank))
+        with pytest.raises(IBError) as e:
+            g.gmres(b)
+        assert e.value.code == abi.IB_E_HIP and "timed out" in str(e.value), (rank, str(e.value))
+        monkeypatch.delenv("IB_GMRES_FAIL_RANK")
+        x, its = g.gmres(b)
+        assert its == want[1] and np.array_equal(x, want[0])
+    g.close()
