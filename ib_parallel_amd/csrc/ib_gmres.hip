@@ -1795,13 +1795,7 @@ size_t gmres_coopw_ws(int nf, int kmax, int P, int R, int NL) {
          (size_t)2 * P + (size_t)(kmax + 1) * kmax + (size_t)3 * kmax + (size_t)P * R * (size_t)std::max(0, kmax + 1 - NL);
 }
 
-// The small form reserves what a Hessenberg copy per workgroup would take:
-// the size by which a caller's fixed workspace admits or refuses a solve.
-size_t gmres_coop_ws(int nf, int kmax, int P) {
-  const size_t reserved =
-      kCoopSyncDoubles + (size_t)P * (kmax + 2) + (size_t)4 * P + (size_t)nf + (size_t)P * (kmax + 1) * kmax;
-  return std::max(reserved, gmres_coopw_ws(nf, kmax, P, 0, kmax + 1));
-}
+size_t gmres_coop_ws(int nf, int kmax, int P) { return gmres_coopw_ws(nf, kmax, P, 0, kmax + 1); }
 
 // the kernel arguments of one solve, its workspace laid out in ws
 static GmCoopWArgs coopw_args(int nf, int kmax, int maxit, int P, int R, int NL, const double* S, const double* b,

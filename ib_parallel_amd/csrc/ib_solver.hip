@@ -8,7 +8,7 @@
 
 // The workspace of ib_op_gmres_noalloc: 16 MiB of device memory per GPU the
 // library runs on, held until the process ends (the airfoil + flap system,
-// nf = 800 at restart 1000, needs 11 MiB).  Host code never passes the
+// nf = 800 at restart 1000, needs 10.8 MiB).  Host code never passes the
 // array's name to a kernel: it stands for no device address on the host.
 constexpr size_t kScratchDoubles = (size_t)2 << 20;
 static __device__ __align__(256) double scratch[kScratchDoubles];

@@ -3,6 +3,8 @@
 workgroups that is not a power of two, the change from direct sums of the
 partial coefficients to published ones, restarts, basis vectors past the LDS,
 an initial guess that already satisfies the tolerance."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -105,3 +107,30 @@ def test_a_workgroup_that_gives_up_fails_the_solve(monkeypatch, npts, form, grou
         x, its = g.gmres(b)
         assert its == want[1] and np.array_equal(x, want[0])
     g.close()
+
+
+def test_workspace_of_the_small_form_is_what_it_lays_out():
+    """nf = 200 at restart 1000, 16 workgroups: one Hessenberg matrix (8 MB) and
+    the exchange buffers (3 x 1001 x 16 values), not a matrix per workgroup.
+    Against a handle of the one-workgroup solve, which keeps no such workspace;
+    4 MB for the allocator's granularity."""
+    from ib_parallel_amd import GpuSim, library
+    hip = library()
+    hip.hipMemGetInfo.argtypes = [C.POINTER(C.c_size_t), C.POINTER(C.c_size_t)]
+
+    def taken(form, groups):
+        free, total = [C.c_size_t() for _ in range(2)], C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(free[0]), C.byref(total)) == 0
+        g = GpuSim(*_circle(100, gmres_restart=1000, gmres_form=form))
+        assert hip.hipMemGetInfo(C.byref(free[1]), C.byref(total)) == 0
+        assert g.gmres_info()[:2] == (form, groups)
+        return g, free[0].value - free[1].value
+
+    for form, groups in ((1, 1), (2, 16)):  # what the runtime takes once
+        taken(form, groups)[0].close()
+    one, base = taken(1, 1)
+    two, mem = taken(2, 16)
+    one.close()
+    two.close()
+    words = 1000 * 1001 + 3 * 1001 * 16 + 4 * 1001 + 4 * 200 + 3 * 1000 + 2 * 16 + 40
+    assert mem - base < 8 * words + (4 << 20), (mem, base)

@@ -86,7 +86,18 @@ def test_noalloc_gmres_equals_op_gmres():
         s.close()
 
 
-def test_noalloc_gmres_refuses():
+def test_noalloc_gmres_of_a_long_restart():
+    """The small form keeps one Hessenberg matrix whatever its number of
+    workgroups: 8 MiB at restart 1000."""
+    from ib_parallel_amd import GpuSim
+    s = GpuSim(*decks.tiny_case(gmres_form=2, gmres_restart=1000))
+    assert s.advance().status == abi.IB_OK
+    assert s.gmres_info()[:2] == (2, 4), s.gmres_info()
+    _pair(s, 1)
+    s.close()
+
+
+def test_noalloc_gmres_refuses(monkeypatch):
     from ib_parallel_amd import GpuSim
 
     def status(sim):
@@ -96,10 +107,13 @@ def test_noalloc_gmres_refuses():
         xd.free()
         return rc
 
-    # the cooperative solve for nf <= 256 at restart 1000 keeps a Hessenberg
-    # matrix per workgroup: 4 x 1001 x 1000 doubles, 32 MB of workspace
-    s = GpuSim(*decks.tiny_case(gmres_form=2, gmres_restart=1000))
-    assert s.gmres_info()[:2] == (2, 4), s.gmres_info()
+    # nf = 1024 at restart 1000 with all but two basis vectors past the LDS:
+    # 1024 x 999 + 1001 x 1000 doubles and the exchange buffers, 16.3 MiB
+    monkeypatch.setenv("IB_COOPW_LDS_VECTORS", "2")
+    p, _ = decks.cylinder_case(m=652, n=652, mgridlev=1, npts=512, tol=1e-11, gmres_restart=1000)
+    s = GpuSim(p, [decks.cylinder_body(512)])
+    monkeypatch.delenv("IB_COOPW_LDS_VECTORS")
+    assert s.gmres_info()[:2] == (3, 32), s.gmres_info()
     assert status(s) == abi.IB_E_INVAL
     assert "static maximum" in s._err(s.h), s._err(s.h)
     s.close()
