@@ -32,6 +32,7 @@ struct HipError : std::runtime_error {
 #define IB_LAUNCH_CHECK() IB_HIP(hipGetLastError())
 
 constexpr int kMaxStages = 24;
+constexpr int kEndsNever = 1, kEndsAlways = 2;
 constexpr int kRegStages = 12;  // the most stages of a pass with register ends
 constexpr int kTaps = 49;  // (2*support2+1)^2, support2 = ceiling(3) (src/grid.F90:12,468)
 
@@ -48,6 +49,7 @@ struct FFTPlan {
   int L, M, N;
   int nst;
   int rad[kMaxStages];
+  int ends;  // register ends (k_dst_xr, k_dst_yr): 0 by rule, kEndsNever, kEndsAlways
   unsigned mLR[kRegStages], mNs[kRegStages];  // division by L/rad[i] and by rad[0] .. rad[i-1]: see div_by
   const double2* W;  // W[t] = exp(-2 pi i t / L), device
 };

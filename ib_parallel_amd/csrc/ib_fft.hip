@@ -797,6 +797,14 @@ static std::vector<int> factorize(int L) {
   return r;
 }
 
+// IB_DST_FORM=fft:staged, fft:ends: see dst_tiles
+static int ends_rule() {
+  const char* f = std::getenv("IB_DST_FORM");
+  if (f && std::strcmp(f, "fft:staged") == 0) return kEndsNever;
+  if (f && std::strcmp(f, "fft:ends") == 0) return kEndsAlways;
+  return 0;
+}
+
 void HostFFTPlan::init(int N) {
   dev.N = N;
   dev.M = N + 1;
@@ -804,6 +812,7 @@ void HostFFTPlan::init(int N) {
   std::vector<int> rad = factorize(dev.L);
   if ((int)rad.size() > kMaxStages) throw HipError("FFT length has too many factors");
   dev.nst = (int)rad.size();
+  dev.ends = ends_rule();
   for (int i = 0, ns = 1; i < dev.nst; ns *= rad[i++]) {
     dev.rad[i] = rad[i];
     if (i >= kRegStages) continue;
@@ -835,13 +844,17 @@ static size_t reg_lds_bytes(const FFTPlan& pl, int nfft) { return (size_t)2 * nf
 // 5.4 matrix cores; 320: 7.7 and 7.6; columns, 200: 10.7 and 10.9); a strided
 // batch is 1.3 times faster without the matrix cores already at 200.
 static bool fft_reg_plan(const FFTPlan& pl, int from) {
-  return !fft_has_generic(pl) && pl.nst >= 2 && pl.nst <= kRegStages && pl.rad[0] == 8 && pl.M >= from;
+  return pl.ends != kEndsNever && !fft_has_generic(pl) && pl.nst >= 2 && pl.nst <= kRegStages && pl.rad[0] == 8 &&
+         (pl.M >= from || pl.ends == kEndsAlways);
 }
 constexpr int kRegRow = 320, kRegCol = 200, kRegBatch = 200;
 // a launch of tiles of `tile` pairs, nfft transforms in all (column passes
 // split an index by the tile with a shift)
 static bool fft_reg_ends(const FFTPlan& pl, int from, int tile, int nfft, size_t max_lds) {
-  return fft_reg_plan(pl, from) && (tile & (tile - 1)) == 0 && reg_lds_bytes(pl, nfft) <= max_lds;
+  const bool ok = fft_reg_plan(pl, from) && (tile & (tile - 1)) == 0 && reg_lds_bytes(pl, nfft) <= max_lds;
+  if (!ok && pl.ends == kEndsAlways)
+    throw HipError("IB_DST_FORM=fft:ends: no pass with register ends for this length and tile");
+  return ok;
 }
 // Threads: about four points each, so that a stage is one or two rounds.  Us per
 // field of a batch of 32, 128 / 256 / 512 threads: columns of 400 points, one
@@ -1052,7 +1065,9 @@ void dst_y(hipStream_t st, const FFTPlan& pl, int mode, const DstLaunch& l, cons
 //
 // IB_DST_TILES=rp,cp forces the Stockham tiles; IB_DST_TUNE=0 keeps the
 // fixed rule (rp 2 up to transform length 512, else 1; cp 1); neither times
-// anything.  IB_DST_FORM=fft keeps the Stockham form, =dense takes the
+// anything.  IB_DST_FORM=fft keeps the Stockham form (=fft:staged without
+// register ends, =fft:ends with them at every length: an error where a pass
+// has none; tests compare the two), =dense takes the
 // matrix-core form for both classes (its fastest configuration, or the
 // (T, KS) = (1, 8) configuration when nothing is timed), =dense:k the matrix-core
 // form in configuration k without timing, =auto (the default) times.
@@ -1095,7 +1110,7 @@ float time_launches(hipStream_t st, F&& launch) {
 int form_rule(int* cfg) {
   const char* f = std::getenv("IB_DST_FORM");
   if (!f || !*f || std::strcmp(f, "auto") == 0) return 0;
-  if (std::strcmp(f, "fft") == 0) return 1;
+  if (std::strcmp(f, "fft") == 0 || ends_rule() != 0) return 1;
   if (std::strcmp(f, "dense") == 0) return 2;
   int k = -1;
   char tail = 0;
@@ -1103,7 +1118,7 @@ int form_rule(int* cfg) {
     *cfg = k;
     return 3;
   }
-  throw HipError("IB_DST_FORM must be fft, dense, dense:k (0 <= k < 5) or auto");
+  throw HipError("IB_DST_FORM must be fft, fft:staged, fft:ends, dense, dense:k (0 <= k < 5) or auto");
 }
 
 struct Scratch {
@@ -1148,7 +1163,7 @@ DstTiles dst_tiles(hipStream_t st, const FFTPlan& px, const FFTPlan& py, const D
     return t;
   }
   const bool try_dense = dense_ok && rule != 1;
-  const std::array<long, 6> key{g.m, g.n, px.L, py.L, (long)max_lds, (long)(rule * 2 + (try_dense ? 1 : 0))};
+  const std::array<long, 6> key{g.m, g.n, px.L, py.L, (long)max_lds, (long)(px.ends * 8 + rule * 2 + (try_dense ? 1 : 0))};
   std::lock_guard<std::mutex> lock(g_tile_mu);
   auto it = g_tiles.find(key);
   if (it != g_tiles.end()) return it->second;
