@@ -413,7 +413,7 @@ struct ib_handle {
     t.begin(st, pass_bytes(mode == X_SUBFROM ? 2 : (mode == X_POINTROT ? 0 : 1), 0, 1, a.batch));
     const int form = cls == 0 ? tiles.xform : tiles.xform_b;
     if (form > 0 && mode != X_POINTROT) dst_dense_x(st, dmx, mode, a, g, form - 1);
-    else dst_x(st, px.dev, mode, a, g, cls == 0 ? tiles.rp : tiles.rp_b, max_lds);
+    else dst_x(st, px.dev, mode, a, g, a.strided ? tiles.rp_b : tiles.rp, max_lds);
     t.end(st);
   }
   void ypass(int mode, const DstLaunch& a) {
@@ -422,7 +422,7 @@ struct ib_handle {
     t.begin(st, pass_bytes(mode == Y_PRED ? 2 : 1, mode == Y_PRED ? 2 : (mode == Y_SCALE2 ? 1 : 0), 1, a.batch));
     const int form = cls == 1 ? tiles.yform : tiles.yform_b;
     if (form > 0) dst_dense_y(st, dmy, mode, a, g, form - 1, tq, (int)(tq.n / (size_t)g.P));
-    else dst_y(st, py.dev, mode, a, g, cls == 1 ? tiles.cp : tiles.cp_b, max_lds);
+    else dst_y(st, py.dev, mode, a, g, a.strided ? tiles.cp_b : tiles.cp, max_lds);
     t.end(st);
   }
 
