@@ -861,10 +861,13 @@ static bool fft_reg_ends(const FFTPlan& pl, int from, int tile, int nfft, size_t
 // pair 2.96 / 2.67 / 4.06; of 512 points, two pairs 10.0 / 7.9 / 7.4; rows of
 // 400 points 1.19 / 1.09 / 1.60; one field's rows of 1024 points 10.4 / 8.6 / 8.1.
 static int reg_threads(const FFTPlan& pl, int nfft) { return nfft * pl.L >= 2048 ? 512 : 256; }
-// Pairs per workgroup of a strided batch: the most that keep it to 1280 points
-// (us per field of 32, rows + columns, 1 / 2 / 4 pairs: 200 points 1.30 / 1.19 /
-// 1.38, 320 x 240 2.25 / 1.78 / 2.19, 400 points 3.76 / 4.32 / 5.53).
-static int reg_batch_tile(const FFTPlan& pl) { return pl.L <= 320 ? 4 : (pl.L <= 640 ? 2 : 1); }
+// Pairs per workgroup of a strided batch: two up to fields of 320 points (L =
+// 640), else one.  Us per field of 314 with one / two pairs: rows of 200 points
+// 0.39 / 0.28, of 320 0.59 / 0.56, of 400 1.09 / 1.26, of 512 1.79 / 1.82; columns
+// of 200 0.85 / 0.58, of 240 1.51 / 1.08, of 400 2.71 / 2.97, of 512 4.50 / 4.04
+// (one number serves both passes).  Four pairs lose everywhere (200 points 0.34
+// and 0.84).
+static int reg_batch_tile(const FFTPlan& pl) { return pl.L <= 640 ? 2 : 1; }
 
 bool fft_has_generic(const FFTPlan& pl) {
   for (int st = 0; st < pl.nst; ++st) {
