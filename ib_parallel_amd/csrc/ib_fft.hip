@@ -361,13 +361,17 @@ __device__ __forceinline__ double row_value(const XArgs& a, const PointPatch& pt
 //  * the twiddles come from the table in memory (L1), not from a copy in LDS,
 //    so a workgroup's LDS holds the two buffers only and a CU more workgroups;
 //  * an index is split by a multiplication (div_by), not a division.
-// What bounds them: a single field has at most 256 workgroups, one round of the
-// chip, and waits on a chain of a dozen barriers and loads; a batch has its
+// What bounds them: a single field has one workgroup per tile of rows or columns
+// (100 for 200 points, 512 for the columns of 1024 x 512), one or two rounds of
+// the chip, and waits on a chain of a dozen barriers and loads; a batch has its
 // instructions, half of them addresses, at five wavefronts per SIMD (89
-// registers).  Us per field, plain form -> this one: one field, rows of 400
-// points 7.9 -> 6.4, of 1024 11.5 -> 8.1, columns of 400 13.3 -> 11.1, of 512
-// 18.7 -> 15.0; a batch of 8 -> of 32 fields, rows of 200 1.13 -> 0.40, of 400
-// 2.29 -> 1.09, columns of 200 1.95 -> 0.79, of 400 4.34 -> 2.67.
+// registers).  Us per field, staged -> this form, the same launch on both sides:
+//   one field         rows of 200 6.8 -> 5.6, 400 7.9 -> 6.4, 1024 11.6 -> 8.2;
+//                     columns of 200 10.8 -> 9.1, 400 13.3 -> 11.0, 512 (of 1023) 18.6 -> 15.3
+//   batch of 8        rows of 400 2.31 -> 1.59, columns 4.31 -> 3.71
+//   batch of 32       rows of 400 1.66 -> 1.19, columns 3.49 -> 2.83
+//   batch of 314      rows of 200 0.43 -> 0.28, 400 1.51 -> 1.09, 512 2.59 -> 1.80;
+//                     columns of 200 1.21 -> 0.58, 400 3.33 -> 2.72, 512 5.92 -> 4.51
 // ------------------------------------------------------------------------
 __device__ __forceinline__ int pd(int i) { return i + (i >> 3); }
 __host__ __device__ inline int pd_len(int L) { return L + (L >> 3) + 1; }
@@ -837,12 +841,17 @@ void HostFFTPlan::release() {
 size_t dst_lds_bytes(const FFTPlan& pl, int nfft) { return (size_t)(2 * nfft + 1) * pl.L * sizeof(double2); }
 
 static size_t reg_lds_bytes(const FFTPlan& pl, int nfft) { return (size_t)2 * nfft * pd_len(pl.L) * sizeof(double2); }
-// Whether a plan takes the passes with register ends: the fixed radices, and
-// above the lengths where a single field goes to the matrix cores instead.
-// There the plain form is what the matrix-core form is timed against, and a
-// faster one would turn near ties (us, one field, 200 points: rows 6.7 plain,
-// 5.4 matrix cores; 320: 7.7 and 7.6; columns, 200: 10.7 and 10.9); a strided
-// batch is 1.3 times faster without the matrix cores already at 200.
+// Whether a plan takes the passes with register ends: the fixed radices, from
+// the lengths below on.  The form is faster at every length tried (us, one field,
+// staged / register ends / matrix cores: rows of 96 points 6.1 / 5.2 / 4.6, 200
+// 6.7 / 5.6 / 5.5, 256 6.6 / 5.7 / 5.7, 288 7.5 / 5.9 / 7.6, 320 7.8 / 6.3 / 7.8;
+// columns of 128 9.4 / 7.7 / 9.2, 192 10.6 / 8.7 / 10.6, 200 10.7 / 9.0 / 10.9).
+// The lengths are there for the results, not for speed: up to 256 points a row
+// pass goes to the matrix cores, which round differently, because they beat the
+// staged pass by the 10% that dst_tiles asks for; against register ends they do
+// not, so the field would change form and its results their last bits.  The
+// lengths stand above the last such grid, which leaves the staged pass to rows of
+// 260 to 319 points and to columns and strided batches below 200.
 static bool fft_reg_plan(const FFTPlan& pl, int from) {
   return pl.ends != kEndsNever && !fft_has_generic(pl) && pl.nst >= 2 && pl.nst <= kRegStages && pl.rad[0] == 8 &&
          (pl.M >= from || pl.ends == kEndsAlways);
@@ -856,10 +865,12 @@ static bool fft_reg_ends(const FFTPlan& pl, int from, int tile, int nfft, size_t
     throw HipError("IB_DST_FORM=fft:ends: no pass with register ends for this length and tile");
   return ok;
 }
-// Threads: about four points each, so that a stage is one or two rounds.  Us per
-// field of a batch of 32, 128 / 256 / 512 threads: columns of 400 points, one
-// pair 2.96 / 2.67 / 4.06; of 512 points, two pairs 10.0 / 7.9 / 7.4; rows of
-// 400 points 1.19 / 1.09 / 1.60; one field's rows of 1024 points 10.4 / 8.6 / 8.1.
+// Threads: 512 from 2048 points in a workgroup's transforms on, else 256 (1.6
+// points each for one transform of a field of 200, 3.1 of 400, 4 of 512 or of 1024,
+// up to 16 for four pairs of predictor columns).  Us per field of a batch of 32,
+// 128 / 256 / 512 threads: columns of 400 points, one pair 2.96 / 2.67 / 4.06; of
+// 512 points, two pairs 10.0 / 7.9 / 7.4; rows of 400 points 1.19 / 1.09 / 1.60;
+// one field's rows of 1024 points 10.4 / 8.6 / 8.1.
 static int reg_threads(const FFTPlan& pl, int nfft) { return nfft * pl.L >= 2048 ? 512 : 256; }
 // Pairs per workgroup of a strided batch: two up to fields of 320 points (L =
 // 640), else one.  Us per field of 314 with one / two pairs: rows of 200 points
