@@ -1427,8 +1427,13 @@ __device__ __forceinline__ void coopw_solve(const GmCoopWArgs& a, int c, unsigne
           gc_wait_stores();  // the clears of the step before
           const int row = RW * q + gw_row<RW>(l);
           if (l < RW && row < Rc) {
+            double* p = a.x3 + cur * nf + r0 + row;
             const double v = gw_mul(ub[r0 + row], inv);
-            xc_put<X2>(a.x3 + cur * nf + r0 + row, (kSmall ? wl[row] : gw_mul(wl[row], inv)) + sum);
+            const double u = (kSmall ? wl[row] : gw_mul(wl[row], inv)) + sum;
+            // once the rows are out, another wavefront may write the next vector
+            // over ub: the read of v is issued before the store
+            asm volatile("" : : "v"(p) : "memory");
+            xc_put<X2>(p, u);
             if (it < NL) Vl[row * NL + it] = v;
             else Vgc[(size_t)row * ldg + (it - NL)] = v;
           }
