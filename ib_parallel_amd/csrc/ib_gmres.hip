@@ -1461,26 +1461,26 @@ __device__ __forceinline__ void coopw_solve(const GmCoopWArgs& a, int c, unsigne
           }
           hv = carry;
         } else {
-        double part = 0.0;  // lane w: the sum over j = 64 w ..
+          double part = 0.0;  // lane w: the sum over j = 64 w ..
 #pragma unroll 1
-        for (int w0 = 0; 64 * w0 <= it; w0 += 4) {
-          double p[4];
+          for (int w0 = 0; 64 * w0 <= it; w0 += 4) {
+            double p[4];
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int j = 64 * (w0 + i) + lane, jj = min(j, it);
-            double al = alpha[jj];
-            const double h = hcol[jj];
-            al = j < it ? -sn * al : cc;
-            if (j <= it) alpha[j] = al;
-            p[i] = j <= it ? gw_mul(al, h) : 0.0;
-          }
+            for (int i = 0; i < 4; ++i) {
+              const int j = 64 * (w0 + i) + lane, jj = min(j, it);
+              double al = alpha[jj];
+              const double h = hcol[jj];
+              al = j < it ? -sn * al : cc;
+              if (j <= it) alpha[j] = al;
+              p[i] = j <= it ? gw_mul(al, h) : 0.0;
+            }
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const double q = gm_wave_sum(p[i]);
-            if (lane == w0 + i) part = q;
+            for (int i = 0; i < 4; ++i) {
+              const double q = gm_wave_sum(p[i]);
+              if (lane == w0 + i) part = q;
+            }
           }
-        }
-        hv = gm_readlane(gm_row_sum16(part), 0);
+          hv = gm_readlane(gm_row_sum16(part), 0);
         }
       }
       if (!kSmall && c == 0) {
@@ -1527,35 +1527,35 @@ __device__ __forceinline__ void coopw_solve(const GmCoopWArgs& a, int c, unsigne
     const int top = it - 1;
     if (c == 0) {
       if constexpr (!kSmall) {
-      double* rc = hcol;   // the rotations (hcol and alpha are free here)
-      double* rsn = alpha;
-      for (int k = gm_opaque(threadIdx.x); k <= top; k += T) {
-        rc[k] = a.rot[3 * k];
-        rsn[k] = a.rot[3 * k + 1];
-      }
-      __syncthreads();
-      // the previous rotations on every column k (thread k), its diagonal
-      // from the step: the rows are read across the columns, eight rows
-      // ahead of the recurrence
-      for (int k = gm_opaque(threadIdx.x); k <= top; k += T) {
-        double* col = a.Ht + k;
-        double carry = col[0];
-        for (int j0 = 0; j0 < k; j0 += 8) {
-          double h[8];
+        double* rc = hcol;   // the rotations (hcol and alpha are free here)
+        double* rsn = alpha;
+        for (int k = gm_opaque(threadIdx.x); k <= top; k += T) {
+          rc[k] = a.rot[3 * k];
+          rsn[k] = a.rot[3 * k + 1];
+        }
+        __syncthreads();
+        // the previous rotations on every column k (thread k), its diagonal
+        // from the step: the rows are read across the columns, eight rows
+        // ahead of the recurrence
+        for (int k = gm_opaque(threadIdx.x); k <= top; k += T) {
+          double* col = a.Ht + k;
+          double carry = col[0];
+          for (int j0 = 0; j0 < k; j0 += 8) {
+            double h[8];
 #pragma unroll
-          for (int i = 0; i < 8; ++i) h[i] = col[(long)min(j0 + i + 1, k) * kmax];
+            for (int i = 0; i < 8; ++i) h[i] = col[(long)min(j0 + i + 1, k) * kmax];
 #pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            const int j = j0 + i;
-            if (j < k) {
-              const double hn = h[i];
-              col[(long)j * kmax] = rc[j] * carry + rsn[j] * hn;
-              carry = -rsn[j] * carry + rc[j] * hn;
+            for (int i = 0; i < 8; ++i) {
+              const int j = j0 + i;
+              if (j < k) {
+                const double hn = h[i];
+                col[(long)j * kmax] = rc[j] * carry + rsn[j] * hn;
+                carry = -rsn[j] * carry + rc[j] * hn;
+              }
             }
           }
+          col[(long)k * kmax] = a.rot[3 * k + 2];
         }
-        col[(long)k * kmax] = a.rot[3 * k + 2];
-      }
       }
       __syncthreads();
       for (int kb1 = top; kb1 >= 0; kb1 -= kCwBlk) {
