@@ -58,7 +58,8 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
-KCLASS = {0: "k_dst_x (row pass, time step)", 1: "k_dst_y (column pass, time step)",
+KCLASS = {0: "k_dst_x (row pass, time step; k_dst_xr with register ends)",
+          1: "k_dst_y (column pass, time step; k_dst_yr with register ends)",
           2: "k_dst_x (batched row pass, Schur assembly)", 3: "k_dst_y (batched column pass, Schur assembly)",
           4: "k_gmres_coopw (one dense GMRES solve over P workgroups of one XCD; "
              "k_gmres_dense in one workgroup where no split fits)"}
@@ -153,7 +154,7 @@ def run_gpu(args):
     roof = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": None}
     roof.update(summary(dom))
-    tr, tk = traffic_for(KCLASS[dom])
+    tr, tk = traffic_for(KCLASS[dom], args.workload)
     roof["traffic"] = tr
     if tr is not None:
         roof["traffic_source"] = f"profiles/pmc_traffic.json ({tk}, FETCH_SIZE + WRITE_SIZE, copy-calibrated)"
@@ -230,7 +231,7 @@ def run_batched(args):
     mode = batch.mode
     tiles = batch.dst_tiles()
     batch.close()
-    plain = [GpuSim(p, b) for p, b in decks.ellipse_batch_cases(count=args.batch)]
+    plain = [GpuSim(p, b) for p, b in cases]
     for s in plain:
         s.advance()
     device_sync()
@@ -253,7 +254,8 @@ def run_batched(args):
         "serial_plain_value": round(vs, 3),
         "serial_plain_ms_per_step": round(ts / args.batch_steps * 1e3, 3),
         "speedup_vs_serial_plain": round(vb / vs, 2), "create_s": round(t_create, 2),
-        "serial_plain": "standalone handles (ib_create), each replaying its captured step graphs",
+        "serial_plain": "standalone handles (ib_create), each " + (
+            "replaying its captured step graphs" if args.batch_launch_mode == 0 else "with plain launches"),
         "fused_dst_tile_rules": dict(zip(("row", "column"), tiles)),
     }
     return res
@@ -556,9 +558,12 @@ def run_dst_compare(args):
     return res
 
 
-def traffic_for(kernel_label):
+def traffic_for(kernel_label, workload):
     """Calibrated HBM bytes per launch of the kernel from the committed
-    counter summary (profiles/pmc_traffic.json), or None."""
+    counter summary (profiles/pmc_traffic.json, taken on the airfoil + flap
+    workload), or None."""
+    if workload != "airfoil_flap":
+        return None, None
     path = os.path.join(ROOT, "profiles", "pmc_traffic.json")
     if not os.path.exists(path):
         return None, None
@@ -704,7 +709,8 @@ def main():
     ap.add_argument("--batch-steps", type=int, default=5)
     ap.add_argument("--batch-only", action="store_true", help="only the batched measurement (one JSON object)")
     ap.add_argument("--batch-launch-mode", type=int, default=0,
-                    help="1: the batched step's launches go to the stream directly instead of a graph replay")
+                    help="1: the launches of the batched and of the serial steps go to the stream directly "
+                         "instead of a graph replay (for traced runs)")
     ap.add_argument("--pmc-copy-mb", type=float, default=0.0,
                     help="run a device-to-device copy of this size first (calibrates counter runs)")
     ap.add_argument("--adjoint-steps", type=int, default=40, help="steps of the adjoint measurement (0: skip)")

@@ -1,5 +1,7 @@
 """bench.py's command line on the CPU: it measures one GPU only and says so,
-before it touches a device, when asked for more."""
+before it touches a device, when asked for more; and the HBM traffic it prints
+is that of the kernel and the workload it was measured on."""
+import json
 import os
 import subprocess
 import sys
@@ -13,3 +15,13 @@ def test_more_than_one_gpu_is_refused_with_a_message():
     assert r.returncode == 2
     assert "one GPU only" in r.stderr
     assert r.stdout == ""
+
+
+def test_traffic_is_that_of_the_measured_workload():
+    sys.path.insert(0, ROOT)
+    import bench
+    with open(os.path.join(ROOT, "profiles", "pmc_traffic.json")) as fh:
+        kernels = json.load(fh)["kernels"]
+    name = "k_gmres_coopw<2, 13>"  # nf = 800: 13 columns of 64 per lane
+    assert bench.traffic_for(bench.KCLASS[4], "airfoil_flap") == (round(kernels[name]["bytes_per_launch"]), name)
+    assert bench.traffic_for(bench.KCLASS[4], "plate") == (None, None)
