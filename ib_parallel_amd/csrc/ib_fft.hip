@@ -849,9 +849,10 @@ static size_t reg_lds_bytes(const FFTPlan& pl, int nfft) { return (size_t)2 * nf
 // The lengths are there for the results, not for speed: up to 256 points a row
 // pass goes to the matrix cores, which round differently, because they beat the
 // staged pass by the 10% that dst_tiles asks for; against register ends they do
-// not, so the field would change form and its results their last bits.  The
-// lengths stand above the last such grid, which leaves the staged pass to rows of
-// 260 to 319 points and to columns and strided batches below 200.
+// not from about 160 points on, so the field would change form and its results
+// their last bits.  The lengths stand above the last such grid, which leaves the
+// staged pass to rows of 260 to 319 points and to columns and strided batches
+// below 200.
 static bool fft_reg_plan(const FFTPlan& pl, int from) {
   return pl.ends != kEndsNever && !fft_has_generic(pl) && pl.nst >= 2 && pl.nst <= kRegStages && pl.rad[0] == 8 &&
          (pl.M >= from || pl.ends == kEndsAlways);

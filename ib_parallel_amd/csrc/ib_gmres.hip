@@ -799,7 +799,7 @@ __device__ __forceinline__ void gc_wait_stores() { asm volatile("s_waitcnt vmcnt
 
 // ------------------------------------------------------------------------
 // The dense solve over P workgroups of one XCD: nf <= 1024 and Krylov spaces
-// of up to 1024 vectors (full GMRES of the airfoil + flap system, nf = 800,
+// of up to 1023 vectors (full GMRES of the airfoil + flap system, nf = 800,
 // restart 1000, over 32 workgroups; the hinged plate, nf = 202, over 4).
 // Workgroup c owns rows [c R, c R + R) of S and of every Krylov vector:
 //  * wavefront q owns RW local rows; lane l holds S[row][l + 64k], k < CQ, in

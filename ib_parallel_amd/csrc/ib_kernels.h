@@ -473,7 +473,7 @@ bool gmres_coop_plan(int nf, int kmax, size_t max_lds, int* P, int* R);
 size_t gmres_coop_ws(int nf, int kmax, int P);
 void gmres_coop(hipStream_t st, int nf, int kmax, int maxit, int P, int R, const double* S, const double* b, double* x,
                 GmresDev* s, double rtol, double atol, double* ws, int xcd, int nxcd);
-// The same kernel's layout for nf <= 1024 and up to 1024 Krylov vectors (S
+// The same kernel's layout for nf <= 1024 and up to 1023 Krylov vectors (S
 // rows in registers, basis rows in LDS up to NL vectors, the rest in HBM);
 // plan: P, rows per workgroup R and NL, false if no split fits.  ws holds
 // gmres_coopw_ws doubles.
