@@ -1423,17 +1423,15 @@ __device__ __forceinline__ void coopw_solve(const GmCoopWArgs& a, int c, unsigne
           }
 #pragma unroll
           for (int i = 0; i < RW; ++i) acc[i] = -acc[i];
+          // this lane's row, read before the wait and the store below: once a
+          // workgroup's rows are out, its polling wavefronts may write the next
+          // vector over ub
+          const int row = RW * q + gw_row<RW>(l), rr = min(row, Rc - 1);
+          const double v = gw_mul(ub[r0 + rr], inv), w = kSmall ? wl[rr] : gw_mul(wl[rr], inv);
           const double sum = gw_reduce_rows<RW>(acc);
           gc_wait_stores();  // the clears of the step before
-          const int row = RW * q + gw_row<RW>(l);
           if (l < RW && row < Rc) {
-            double* p = a.x3 + cur * nf + r0 + row;
-            const double v = gw_mul(ub[r0 + row], inv);
-            const double u = (kSmall ? wl[row] : gw_mul(wl[row], inv)) + sum;
-            // once the rows are out, another wavefront may write the next vector
-            // over ub: the read of v is issued before the store
-            asm volatile("" : : "v"(p) : "memory");
-            xc_put<X2>(p, u);
+            xc_put<X2>(a.x3 + cur * nf + r0 + row, w + sum);
             if (it < NL) Vl[row * NL + it] = v;
             else Vgc[(size_t)row * ldg + (it - NL)] = v;
           }
